@@ -21,7 +21,6 @@
 #include "mose_internal.h"
 #include "mose_chem.hpp"
 #include "mose_kernels.hpp"
-#include "mose_radau.hpp"
 #include "mose_stage.hpp"
 
 using namespace mose;
@@ -1259,7 +1258,6 @@ extern "C" int mose_pow_batch(mose_ctx* ctx, int64_t n, const double* x, const d
 }
 
 namespace {
-constexpr int kChemTeamsPerWg = TeamShape<9>::per_wg;   // the kernels are instantiated for 9 species
 struct ChemObj {
   ChemDev M{};
   void* tabs = nullptr;          // device copies of the mechanism tables (one allocation)
@@ -1269,7 +1267,7 @@ struct ChemObj {
   int* nstep = nullptr;
   unsigned long long* ctr = nullptr;   // [0] queue, [1..6] stats
   int64_t cap = 0, n = 0;
-  int grid = 0, cus = 0;
+  int cus = 0;
   hipEvent_t ev[2] = {nullptr, nullptr};
   bool valid = false;
 };
@@ -1329,7 +1327,10 @@ extern "C" int mose_chem_create(mose_ctx* ctx, const mose_mechanism* m, int64_t 
   const int ns = m->ns, rows = m->tmax - m->tmin + 1, nr = m->n_arrh + m->n_troe + m->n_lind;
   size_t n_thermo = (size_t)ns * rows, n_st = (size_t)nr * (ns + 1), n_kf = (size_t)m->n_arrh * rows;
   size_t n_troe = (size_t)m->n_troe * 4 * rows, n_lind = (size_t)m->n_lind * 3 * rows;
-  size_t total = 2 * n_thermo + 3 * n_st + 2 * n_kf + n_troe + n_lind + 8;
+  // the two-round mechanisms' tables by temperature (ChemDev::lanes)
+  const bool two = chem_two_rounds(ns, m->n_arrh, nr, m->ni1, m->ni2);
+  const int lcol = two ? (2 * (3 * (ns + 1) + ns) + 15) / 16 * 16 : 0;
+  size_t total = 2 * n_thermo + 3 * n_st + 2 * n_kf + n_troe + n_lind + 8 + (size_t)lcol * rows + 16;
   HIPCHK(ctx, hipMalloc(&o->tabs, total * sizeof(double)));
   double* p = (double*)o->tabs;
   auto put = [&](const double* src, size_t cnt) -> double* {
@@ -1345,12 +1346,41 @@ extern "C" int mose_chem_create(mose_ctx* ctx, const mose_mechanism* m, int64_t 
   M.ni1 = put(m->ni1, n_st); M.ni2 = put(m->ni2, n_st); M.eps = put(m->eps, n_st);
   M.kf = put(m->kf, n_kf); M.kb = put(m->kb, n_kf);
   M.troe = put(m->troe, n_troe); M.lind = put(m->lind, n_lind);
+  M.two_rounds = two ? 1 : 0;
+  M.lcol = lcol;
+  M.lanes = nullptr;
+  if (two) {
+    std::vector<int> ord(nr);
+    chem_order(ns, m->n_arrh, nr, m->ni1, ord.data());
+    std::vector<double> lanes((size_t)lcol * rows, 0.0);
+    auto column = [&](int col, const double* src) {
+      for (int t = 0; t < rows; ++t) lanes[(size_t)t * lcol + col] = src[t];
+    };
+    for (int i = 0; i < nr; ++i) {
+      const int q = ord[i], nz = ns + 1;
+      if (q < m->n_arrh) {
+        column(2 * i, m->kf + (size_t)q * rows);
+        column(2 * i + 1, m->kb + (size_t)q * rows);
+      } else {
+        const bool troe = q < m->n_arrh + m->n_troe;
+        const double* tb = troe ? m->troe + (size_t)(q - m->n_arrh) * 4 * rows
+                                : m->lind + (size_t)(q - m->n_arrh - m->n_troe) * 3 * rows;
+        column(2 * i, tb);
+        column(2 * i + 1, tb + rows);
+        column(2 * (2 * nz + i), tb + 2 * (size_t)rows);
+        if (troe) column(2 * (2 * nz + i) + 1, tb + 3 * (size_t)rows);
+      }
+    }
+    for (int sp = 0; sp < ns; ++sp) {
+      column(2 * (3 * (ns + 1) + sp), m->h + (size_t)sp * rows);
+      column(2 * (3 * (ns + 1) + sp) + 1, m->cp + (size_t)sp * rows);
+    }
+    p = (double*)(((uintptr_t)p + 127) & ~(uintptr_t)127);
+    M.lanes = put(lanes.data(), lanes.size());
+  }
   HIPCHK(ctx, hipGetLastError());
   int cus = 0;
   HIPCHK(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
-  // persistent grid of 256-lane workgroups (24 teams of 10 lanes, one cell per team at a time): enough to give
-  // every SIMD several waves
-  o->grid = (int)std::min<int64_t>((ncell_max + kChemTeamsPerWg - 1) / kChemTeamsPerWg, (int64_t)cus * 8);
   o->cus = cus;
   o->cap = ncell_max;
   const int nz = ns + 1;
@@ -1427,10 +1457,8 @@ static int chem_run(mose_ctx* ctx, ChemObj* o, ChemArgs& A, unsigned long long* 
   hipStream_t s = ctx->stream;
   A.queue = ctr; A.stats = ctr + 1;
   k_zero_u64<<<1, 64, 0, s>>>(ctr, kScratchWords);
-  int grid = (int)std::min<int64_t>((int64_t)o->cus * 8, (A.ncell + kChemTeamsPerWg - 1) / kChemTeamsPerWg);
   HIPCHK(ctx, hipEventRecord(o->ev[0], s));
-  if (method == MOSE_ODE_RADAU5) k_radau<9><<<grid, 256, 0, s>>>(o->M, A);
-  else k_chem<9><<<grid, 256, 0, s>>>(o->M, A);
+  launch_chem(o->M, A, method == MOSE_ODE_RADAU5, o->cus, s);
   HIPCHK(ctx, hipGetLastError());
   HIPCHK(ctx, hipEventRecord(o->ev[1], s));
   unsigned long long st[7];
@@ -1523,9 +1551,7 @@ static int case_chem_launch(mose_ctx* ctx, Case& c, hipStream_t s) {
   A.state = c.P0; A.stride = c.NC; A.dtp = c.dt;
   A.queue = c.chem_ctr; A.stats = c.chem_ctr + 8;
   k_zero_u64<<<1, 64, 0, s>>>(c.chem_ctr, 1);
-  const int grid = (int)std::min<int64_t>((int64_t)o->cus * 8, (A.ncell + kChemTeamsPerWg - 1) / kChemTeamsPerWg);
-  if (c.chem_method == MOSE_ODE_RADAU5) k_radau<9><<<grid, 256, 0, s>>>(o->M, A);
-  else k_chem<9><<<grid, 256, 0, s>>>(o->M, A);
+  launch_chem(o->M, A, c.chem_method == MOSE_ODE_RADAU5, o->cus, s);
   HIPCHK(ctx, hipGetLastError());
   return MOSE_OK;
 }
@@ -1619,10 +1645,8 @@ extern "C" int mose_case_chem_advance(mose_ctx* ctx, int id, double dt, mose_che
   A.state = c->P0; A.stride = c->NC; A.dtp = nullptr; A.dt = dt;
   A.queue = c->chem_ctr; A.stats = c->chem_ctr + 8;
   k_zero_u64<<<1, 64, 0, s>>>(c->chem_ctr, 16);
-  const int grid = (int)std::min<int64_t>((int64_t)o->cus * 8, (A.ncell + kChemTeamsPerWg - 1) / kChemTeamsPerWg);
   HIPCHK(ctx, hipEventRecord(c->ev[1], s));
-  if (c->chem_method == MOSE_ODE_RADAU5) k_radau<9><<<grid, 256, 0, s>>>(o->M, A);
-  else k_chem<9><<<grid, 256, 0, s>>>(o->M, A);
+  launch_chem(o->M, A, c->chem_method == MOSE_ODE_RADAU5, o->cus, s);
   HIPCHK(ctx, hipGetLastError());
   HIPCHK(ctx, hipEventRecord(c->ev[2], s));
   HIPCHK(ctx, hipMemcpyAsync(c->stage_chem, c->chem_ctr + 8, 6 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
