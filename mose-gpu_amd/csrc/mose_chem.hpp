@@ -198,7 +198,7 @@ __device__ __forceinline__ int tshi(int v, int src) { return __shfl(v, src, 64);
 
 // Compact form of the mechanism's reactions, built once per workgroup in LDS: the orders nu'(q, s) and nu''(q, s)
 // as 4-bit fields when every one is an integer in [0, 8] (the powers of both rate classes are then integer powers:
-// (int)rint(nu) for the Arrhenius class, the integral branch of rpow for the falloff classes), the third-body flag
+// nint(nu) for the Arrhenius class, the integral branch of rpow for the falloff classes), the third-body flag
 // (nu'(q, ns+1) > 0) and the third-body efficiencies.  Reactions run in rounds of one per lane: ord lists them with
 // the falloff reactions first, then the other third-body ones, so that the rounds after the first skip both (the
 // rates go to their own places, the order of evaluation does not enter).
@@ -378,8 +378,8 @@ __device__ __forceinline__ double net_rate(const ChemDev& M, const RxnLds& X, in
     for (int s = 0; s < NS; ++s) {
       const double a = n1[s], b = n2[s];
       if (!falloff) {
-        if (a != 0) pf = pf * chem_ipow(coi[s], (int)rint(a));
-        if (b != 0) pr = pr * chem_ipow(coi[s], (int)rint(b));
+        if (a != 0) pf = pf * chem_ipow(coi[s], (int)round(a));
+        if (b != 0) pr = pr * chem_ipow(coi[s], (int)round(b));
       } else {
         if (a != 0) pf = pf * rpow(coi[s], a);
         if (b != 0) pr = pr * rpow(coi[s], b);

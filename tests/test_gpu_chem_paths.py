@@ -71,6 +71,7 @@ MECHS = {
     "13-third-body": all_third_body,
     "order-3": lambda: with_rows([ordered(0, H=2.0)]),
     "four-species": lambda: with_rows([ordered(0, OH=1.0, H2O=1.0)]),
+    "half-order": lambda: with_rows([ordered(1, O=0.5)]),
 }
 
 
