@@ -134,11 +134,12 @@ __device__ __forceinline__ void bc_wall_visc(const mose_dtab& T, const double* P
 
 // BC_Symmetry_Visc (Lib_BC.f90:741-861): the viscous stress of a symmetry face.  The velocity gradient takes the cell
 // and its mirror image across the face along the normal, and along each transverse direction the two neighbours and
-// their mirror images (stencil of the Fm cases :783-802).  sb, sc: the row strides of the transverse directions b, c.
+// their mirror images (stencil of the Fm cases :783-802).  vn: the velocities of the neighbours -b, +b, -c, +c (Vel3,
+// Vel4, Vel7, Vel8); bc_sym_visc reads them at the row strides sb, sc of the transverse directions.
 template <int NS, int NR>
-__device__ __forceinline__ void bc_sym_visc(const mose_dtab& T, const double* P, int64_t NC, const double* m,
-                                            const RecCells& rc, int64_t sb, int64_t sc, double nx, double ny,
-                                            double nz, double area, double* e2) {
+__device__ __forceinline__ void bc_sym_visc_n(const mose_dtab& T, const double* P, int64_t NC, const double* m,
+                                              const RecCells& rc, const double (*vn)[3], double nx, double ny,
+                                              double nz, double area, double* e2) {
   using V = Vars<NS, NR>;
   const int modfm2 = 1 - 2 * rc.modfm;
   const int a = rc.dir - 1, b = rc.dir == 1 ? 1 : 0, c = rc.dir == 3 ? 1 : 2;
@@ -153,15 +154,9 @@ __device__ __forceinline__ void bc_sym_visc(const mose_dtab& T, const double* P,
   double Tk = Pb[V::np] / (rho * Rg), mil, kl;
   int Ti = ftrunc(Tk);
   wilke<NS>(T, Pb, rho, Ti, Tk - Ti, mil, kl);
-  // Vel3, Vel4 (direction b) and Vel7, Vel8 (direction c), then the mirror images Vel5, Vel6, Vel9, Vel10
-  const int64_t nbr[4] = {rc.c - sb, rc.c + sb, rc.c - sc, rc.c + sc};
-  double v1[3], v2[3], vn[4][3], vm[4][3];
+  double v1[3], v2[3], vm[4][3];
 #pragma unroll
   for (int q = 0; q < 3; ++q) v1[q] = Pb[V::nu + q];
-#pragma unroll
-  for (int n = 0; n < 4; ++n)
-#pragma unroll
-    for (int q = 0; q < 3; ++q) vn[n][q] = P[(V::nu + q) * NC + nbr[n]];
   const double d1 = v1[0] * nx + v1[1] * ny + v1[2] * nz;
   v2[0] = v1[0] - 2.0 * d1 * nx;
   v2[1] = v1[1] - 2.0 * d1 * ny;
@@ -195,6 +190,20 @@ __device__ __forceinline__ void bc_sym_visc(const mose_dtab& T, const double* P,
 #pragma unroll
   for (int q = 0; q < 3; ++q) e2[V::nu + q] = -((double)modfm2 * area * St[q]);
   e2[V::np] = -((double)modfm2 * area * (u0 * St[0] + u1 * St[1] + u2 * St[2]));
+}
+
+template <int NS, int NR>
+__device__ __forceinline__ void bc_sym_visc(const mose_dtab& T, const double* P, int64_t NC, const double* m,
+                                            const RecCells& rc, int64_t sb, int64_t sc, double nx, double ny,
+                                            double nz, double area, double* e2) {
+  using V = Vars<NS, NR>;
+  const int64_t nbr[4] = {rc.c - sb, rc.c + sb, rc.c - sc, rc.c + sc};
+  double vn[4][3];
+#pragma unroll
+  for (int n = 0; n < 4; ++n)
+#pragma unroll
+    for (int q = 0; q < 3; ++q) vn[n][q] = P[(V::nu + q) * NC + nbr[n]];
+  bc_sym_visc_n<NS, NR>(T, P, NC, m, rc, vn, nx, ny, nz, area, e2);
 }
 
 // the flux of a far-field face from its face state (the tails of BC_Outflow :1218-1242 and BC_Subsonic_Inflow

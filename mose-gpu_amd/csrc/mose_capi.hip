@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -15,11 +16,13 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "mose_gpu.h"
 #include "mose_internal.h"
 #include "mose_chem.hpp"
+#include "mose_bc.hpp"
 #include "mose_kernels.hpp"
 #include "mose_stage.hpp"
 
@@ -65,6 +68,14 @@ struct Case {
   int ntiles = 0, tiles_cap = 0;
   unsigned long long* dtnext = nullptr;
   bool dt_valid = false;
+  // the planned boundary kernel of the fused paths (k_bc) for the records that act in every stage; ndead others have
+  // their ghosts filled at a download (bc_dead).  nplan = 0: the case runs k_ghost and k_bcrec
+  BcPlan* dplan = nullptr;
+  BcNbr* dnbr = nullptr;
+  double* dgeo = nullptr;         // [8 or 17][nplan]
+  int* drecof = nullptr;
+  int nplan = 0, ndead = 0;
+  bool dead_stale = false;
   // residual norm of the last step (per-workgroup partials of the last stage) and the state hash slots
   double* rpart = nullptr;
   int64_t rpart_cap = 0, nparts_last = 0;
@@ -236,6 +247,9 @@ static void case_free(Case* c) {
   c->rpart_cap = 0;
   if (c->dtiles) (void)hipFree(c->dtiles);
   c->dtiles = nullptr;
+  if (c->dplan) (void)hipFree(c->dplan);
+  c->dplan = nullptr;
+  c->nplan = c->ndead = 0;
   if (c->chem_rows) (void)hipFree(c->chem_rows);
   c->chem_rows = nullptr;
   if (c->stage_chem) (void)hipHostFree(c->stage_chem);
@@ -400,7 +414,152 @@ static size_t case_bytes(const Case& c) {
   b += (std::max<size_t>(c.ff.size(), 1) * sizeof(mose_farfield) + 255) / 256 * 256;
   b += ((size_t)std::max<int64_t>(c.NBP, 1) + 255) / 256 * 256;
   b += 64 * sizeof(double) + 256 + 512;
+  b += c.rec.size() * (sizeof(BcPlan) + sizeof(BcNbr) + (c.sc.viscous ? BCG_VISCOUS : BCG_INVISCID) * d) +
+       (size_t)c.NBP * sizeof(int) + 256;   // the boundary plan (its own allocation)
   return b;
+}
+
+// Inviscid cases read no ghost behind the no-flux faces of a direction of one cell: such records are not planned, and
+// their ghosts are filled (with the others, by k_ghost) when the state is downloaded.  On a 1023^2 Riemann problem they
+// are 2.09 of the 2.10 million records, and took a third of a step.
+static bool bc_dead(const Case& c, const mose_bc_record& r) {
+  const mose_blk& B = c.blk[r.b];
+  const int d = (r.f + 1) / 2;
+  return !c.sc.viscous && r.typ == MOSE_BC_NONE && (d == 1 ? B.n1 : (d == 2 ? B.n2 : B.n3)) == 1;
+}
+
+// f(first, last) over [0, n) in the host's threads (the plan of a large case: 0.3 us a record)
+template <class F>
+static void host_parallel(size_t n, F f) {
+  const size_t parts = n < 32768 ? 1 : std::min<size_t>(8, std::max(1u, std::thread::hardware_concurrency()));
+  std::vector<std::thread> th;
+  for (size_t t = 1; t < parts; ++t) th.emplace_back(f, n * t / parts, n * (t + 1) / parts);
+  f((size_t)0, n / parts);
+  for (auto& t : th) t.join();
+}
+
+static CaseDev make_dev(mose_ctx* ctx, Case& c, const double* Pin, double* Pout);
+static inline unsigned nblocks(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
+
+// The boundary plan (mose_bc.hpp).  Cases of nine species and connections whose transverse maps are not one step along
+// one axis keep k_ghost and k_bcrec (ghost1 forms the first ghost layer next to a cell, no corner).
+static int plan_boundary(mose_ctx* ctx, Case& c, hipStream_t s) {
+  if (c.sc.nsc > 4 || c.rec.empty() || c.NC > 0x7fffffff || std::max({c.NF1, c.NF2, c.NF3, c.NBP}) > 0x7fffffff) return MOSE_OK;
+  auto row_of = [&](int b, const int* x) {
+    const mose_blk& B = c.blk[b];
+    return B.boff + (x[0] + MOSE_GC - 1) + (int64_t)(x[1] + MOSE_GC - 1) * B.pi + (int64_t)(x[2] + MOSE_GC - 1) * B.pi * B.pj;
+  };
+  auto place = [&](int b, int f, const int* x) {
+    const mose_blk& B = c.blk[b];
+    return B.bpoff[f - 1] + (f <= 2 ? (x[1] - 1) + (int64_t)B.n2 * (x[2] - 1)
+                             : f <= 4 ? (x[0] - 1) + (int64_t)B.n1 * (x[2] - 1)
+                                      : (x[0] - 1) + (int64_t)B.n1 * (x[1] - 1));
+  };
+  auto extent = [&](const mose_bc_record& r) {
+    const mose_blk& B = c.blk[r.b];
+    return r.f <= 2 ? B.n1 : (r.f <= 4 ? B.n2 : B.n3);
+  };
+  auto cubic = [&](const mose_bc_record& r) {
+    return (r.typ == MOSE_BC_EXTRAPOLATION && extent(r) >= 3) || r.typ == MOSE_BC_WALL_ADIABATIC ||
+           r.typ == MOSE_BC_WALL_ISOTHERMAL;
+  };
+  // the order: by type, direction and side (the low bits of meta), the records of each in their own order
+  auto key = [&](const mose_bc_record& r) {
+    return (unsigned)r.typ | (unsigned)((r.f + 1) / 2 - 1) << BCP_DIR | (unsigned)(r.f % 2) << BCP_ODD;
+  };
+  std::vector<int> order(c.rec.size(), -1), count(128, 0);
+  for (const auto& r : c.rec)
+    if (!bc_dead(c, r)) ++count[key(r)];
+  for (int q = 0, at = 0; q < 128; ++q) { const int n = count[q]; count[q] = at; at += n; }
+  size_t nlive = 0;
+  for (size_t e = 0; e < c.rec.size(); ++e)
+    if (!bc_dead(c, c.rec[e])) { order[e] = count[key(c.rec[e])]++; ++nlive; }
+  if (nlive == 0) return MOSE_OK;
+  const bool visc = c.sc.viscous != 0;
+  std::vector<int> recof(visc ? (size_t)std::max<int64_t>(c.NBP, 1) : 1, 0);
+  if (visc)
+    host_parallel(c.rec.size(), [&](size_t e0, size_t e1) {
+      for (size_t e = e0; e < e1; ++e) {
+        const int x[3] = {c.rec[e].i, c.rec[e].j, c.rec[e].k};
+        recof[place(c.rec[e].b, c.rec[e].f, x)] = (int)e;
+      }
+    });
+  // the neighbour of cell x of block b one step sg along axis a: its row; behind a boundary face the row that the face's
+  // record copies, or -(place) - 1 where the record mirrors or extrapolates
+  auto neighbour = [&](int b, const int* x, int a, int sg) -> int {
+    const mose_blk& B = c.blk[b];
+    const int n[3] = {B.n1, B.n2, B.n3};
+    int y[3] = {x[0], x[1], x[2]};
+    y[a] += sg;
+    if (y[a] >= 1 && y[a] <= n[a]) return (int)row_of(b, y);
+    const int64_t at = place(b, 2 * a + (sg < 0 ? 1 : 2), x);
+    const mose_bc_record& r = c.rec[recof[at]];
+    if (r.typ == MOSE_BC_CONNECTION) {
+      const int z[3] = {r.is, r.js, r.ks};
+      return (int)row_of(r.bs, z);
+    }
+    if (r.typ == MOSE_BC_SYMMETRY || cubic(r)) return (int)(-at - 1);
+    return (int)row_of(b, x);
+  };
+  std::vector<BcPlan> plan(nlive);
+  std::vector<BcNbr> nbr(visc ? nlive : 0);
+  std::atomic<bool> fits{true};
+  host_parallel(c.rec.size(), [&](size_t e0, size_t e1) {
+    for (size_t e = e0; e < e1; ++e) {
+      if (order[e] < 0) continue;
+      const mose_bc_record& r = c.rec[e];
+      const mose_blk& B = c.blk[r.b];
+      const int at[3] = {r.i, r.j, r.k}, d = (r.f + 1) / 2 - 1, odd = r.f % 2;
+      BcPlan p{};
+      BcNbr nb{};
+      p.c = (int)row_of(r.b, at);
+      p.pos = (int)place(r.b, r.f, at);
+      p.fg = (int)(d == 0 ? B.f1off + (r.i - odd) + (int64_t)(B.n1 + 1) * ((r.j - 1) + (int64_t)B.n2 * (r.k - 1))
+                   : d == 1 ? B.f2off + (r.i - 1) + (int64_t)B.n1 * ((r.j - odd) + (int64_t)(B.n2 + 1) * (r.k - 1))
+                            : B.f3off + (r.i - 1) + (int64_t)B.n1 * ((r.j - 1) + (int64_t)B.n2 * (r.k - odd)));
+      p.e = (int)e;
+      p.b = r.b;
+      p.bs = r.typ == MOSE_BC_CONNECTION ? r.bs : r.b;
+      const int ax[2] = {d == 0 ? 1 : 0, d == 2 ? 1 : 2};
+      unsigned m = key(r);
+      if (r.typ == MOSE_BC_EXTRAPOLATION || r.typ == MOSE_BC_FARFIELD || r.typ == MOSE_BC_NONE) m |= 1u << BCP_ZG;
+      if (cubic(r)) m |= 1u << BCP_CUB;
+      const bool nbrs = visc && (r.typ == MOSE_BC_CONNECTION || r.typ == MOSE_BC_SYMMETRY);
+      for (int q = 0; nbrs && q < 4; ++q) nb.r[q] = neighbour(r.b, at, ax[q / 2], q % 2 ? 1 : -1);
+      if (r.typ == MOSE_BC_CONNECTION) {
+        const int sat[3] = {r.is, r.js, r.ks}, sd = (r.fs + 1) / 2 - 1;
+        const int sax[2] = {sd == 0 ? 1 : 0, sd == 2 ? 1 : 2}, map[2][2] = {{r.d11, r.d12}, {r.d21, r.d22}};
+        p.src = (int)row_of(r.bs, sat);
+        m |= ((unsigned)sd | (r.fs % 2 ? 0u : 4u)) << BCP_IN;
+        for (int t = 0; nbrs && t < 2; ++t) {
+          if (std::abs(map[t][0]) + std::abs(map[t][1]) != 1) { fits = false; return; }
+          const int q = map[t][0] != 0 ? 0 : 1;
+          nb.r[4 + 2 * t] = neighbour(r.bs, sat, sax[q], -map[t][q]);
+          nb.r[5 + 2 * t] = neighbour(r.bs, sat, sax[q], map[t][q]);
+        }
+      }
+      for (int q = 0; q < 8; ++q) m |= (unsigned)(nb.r[q] < 0) << (BCP_EDGE + q);
+      p.meta = (int)m;
+      plan[order[e]] = p;
+      if (visc) nbr[order[e]] = nb;
+    }
+  });
+  if (!fits) return MOSE_OK;
+  c.nplan = (int)nlive;
+  c.ndead = (int)(c.rec.size() - nlive);
+  const size_t pb = plan.size() * sizeof(BcPlan), qb = nbr.size() * sizeof(BcNbr);
+  const size_t gb = plan.size() * (c.sc.viscous ? BCG_VISCOUS : BCG_INVISCID) * sizeof(double);
+  HIPCHK(ctx, hipMalloc(&c.dplan, pb + qb + gb + recof.size() * sizeof(int)));
+  c.dnbr = (BcNbr*)((char*)c.dplan + pb);
+  c.dgeo = (double*)((char*)c.dplan + pb + qb);
+  c.drecof = (int*)((char*)c.dplan + pb + qb + gb);
+  HIPCHK(ctx, hipMemcpyAsync(c.dplan, plan.data(), pb, hipMemcpyHostToDevice, s));
+  if (qb) HIPCHK(ctx, hipMemcpyAsync(c.dnbr, nbr.data(), qb, hipMemcpyHostToDevice, s));
+  HIPCHK(ctx, hipMemcpyAsync(c.drecof, recof.data(), recof.size() * sizeof(int), hipMemcpyHostToDevice, s));
+  k_bc_geometry<<<nblocks((int64_t)plan.size(), 64), 64, 0, s>>>(make_dev(ctx, c, c.P0, c.PA), c.dplan, (int)plan.size(), c.dgeo);
+  HIPCHK(ctx, hipGetLastError());
+  HIPCHK(ctx, hipStreamSynchronize(s));
+  return MOSE_OK;
 }
 
 extern "C" int mose_case_bytes(const mose_scheme* sc, int nb, const int* dims, int nrec, int64_t* bytes) {
@@ -584,7 +743,8 @@ extern "C" int mose_case_create(mose_ctx* ctx, const mose_scheme* sc, int nb, co
     c->path = MOSE_PATH_PLAIN;   // the smoothing needs the whole residual: the per-block launches
   }
   HIPCHK(ctx, hipStreamSynchronize(s));
-  rc = ensure_rpart(ctx, *c, plain_parts(*c));
+  rc = plan_boundary(ctx, *c, s);
+  if (rc == MOSE_OK) rc = ensure_rpart(ctx, *c, plain_parts(*c));
   if (rc != MOSE_OK) { case_free(c.get()); return rc; }
   c->valid = true;
   {
@@ -614,14 +774,21 @@ extern "C" int mose_state_upload(mose_ctx* ctx, int id, const double* P) {
   HIPCHK(ctx, hipMemcpyAsync(c->P0, P, n, hipMemcpyHostToDevice, c->stream));
   HIPCHK(ctx, hipStreamSynchronize(c->stream));
   c->dt_valid = false;
+  c->dead_stale = false;
   return MOSE_OK;
 }
+
+static int fill_dead_ghosts(mose_ctx* ctx, Case& c);
 
 extern "C" int mose_state_download(mose_ctx* ctx, int id, double* P) {
   Case* c = get_case(ctx, id);
   if (!c || !P) return MOSE_ERR_ARG;
   HIPCHK(ctx, hipSetDevice(ctx->device));
   size_t n = (size_t)c->NC * c->nprim * sizeof(double);
+  {
+    const int rc = fill_dead_ghosts(ctx, *c);
+    if (rc != MOSE_OK) return rc;
+  }
   HIPCHK(ctx, hipMemcpyAsync(P, c->P0, n, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(ctx, hipStreamSynchronize(c->stream));
   return MOSE_OK;
@@ -647,16 +814,65 @@ static CaseDev make_dev(mose_ctx* ctx, Case& c, const double* Pin, double* Pout)
   return D;
 }
 
-static inline unsigned nblocks(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
+
+// The start of a step: dt from the slot that the last stage of the step before (or k_dt) left, its place in the history
+// (a device-side position, so that the same launch serves eager and graph steps), and the slot ready for this step's
+// last stage.  The plain path's slot is not its next dt's: dtnext null keeps dt.
+__global__ void k_step_begin(unsigned long long* dtnext, double* dt, double* hist, int* pos, int cap) {
+  if (threadIdx.x == 0 && blockIdx.x == 0) {
+    if (dtnext) {
+      *dt = __longlong_as_double((long long)*dtnext);
+      *dtnext = (unsigned long long)__double_as_longlong(1e5);
+    }
+    int t = *pos;
+    if (t < cap) hist[t] = *dt;
+    *pos = t + 1;
+  }
+}
+
+// The boundary of a fused stage: the planned kernel, or the ghost and the record kernel.  begin: the step's first stage
+// (dt, its history and the slot of the next dt, see StepBegin).
+template <int NS, int NR>
+static void launch_boundary(Case& c, const CaseDev& D, hipStream_t s, bool begin) {
+  if constexpr (NS <= 4) {
+    if (c.nplan > 0) {
+      const StepBegin B{begin ? c.dtnext : nullptr, c.dt, c.dthist, c.histpos, c.hist_cap};
+      const unsigned wgs = nblocks(c.nplan, 64);
+      k_bc<NS, NR><<<D.visc ? 2 * ((wgs + 7) / 8 * 8) : wgs, 64, 0, s>>>(D, c.dplan, c.dnbr, c.nplan, c.drecof, c.dgeo,
+                                                                         c.nplan, B);
+      return;
+    }
+  }
+  if (begin) k_step_begin<<<1, 64, 0, s>>>(c.dtnext, c.dt, c.dthist, c.histpos, c.hist_cap);
+  const int nrec = (int)c.rec.size();
+  if (nrec > 0) {
+    k_ghost<NS, NR><<<nblocks(nrec, 256), 256, 0, s>>>(D);
+    k_bcrec<NS, NR><<<nblocks(nrec, 128), 128, 0, s>>>(D);
+  }
+}
+
+template <int NS, int NR>
+static void launch_ghosts(Case& c, const CaseDev& D, hipStream_t s) {
+  k_ghost<NS, NR><<<nblocks((int64_t)c.rec.size(), 256), 256, 0, s>>>(D);
+}
+
+static int fill_dead_ghosts(mose_ctx* ctx, Case& c) {
+  if (!c.dead_stale || c.ndead == 0) return MOSE_OK;
+  CaseDev D = make_dev(ctx, c, c.P0, c.PA);
+  MOSE_DISPATCH(c.sc, launch_ghosts, c, D, c.stream);
+  HIPCHK(ctx, hipGetLastError());
+  c.dead_stale = false;
+  return MOSE_OK;
+}
 
 template <int NS, int NR>
 static void launch_dt(Case& c, const CaseDev& D, hipStream_t s, int step_index) {
-  k_dt_init<<<1, 64, 0, s>>>(c.dtmin);
+  k_dt_init<<<1, 64, 0, s>>>(D.dtmin);
   for (int b = 0; b < c.nb; ++b) {
     int64_t n = (int64_t)c.blk[b].n1 * c.blk[b].n2 * c.blk[b].n3;
     k_dt<NS, NR><<<nblocks(n, 256), 256, 0, s>>>(D, b);
   }
-  k_dt_final<<<1, 64, 0, s>>>(c.dtmin, c.dt, step_index >= 0 ? c.dthist : nullptr, step_index);
+  k_dt_final<<<1, 64, 0, s>>>(D.dtmin, c.dt, step_index >= 0 ? c.dthist : nullptr, step_index);
 }
 
 template <int NS, int NR>
@@ -794,16 +1010,6 @@ static void launch_stage(Case& c, const CaseDev& D, hipStream_t s, double rkc, b
   else launch_stage_tiles<NS, NR>(D, A, c.sc.riemann, c.sc.viscous != 0, grid, lds, s);
 }
 
-// records the step's dt in the history at the device-side position (the same kernel serves eager and graph steps)
-__global__ void k_step_begin(const double* dt, double* hist, int* pos, int cap) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    int t = *pos;
-    if (t < cap) hist[t] = *dt;
-    *pos = t + 1;
-  }
-}
-
-
 static int case_chem_launch(mose_ctx* ctx, Case& c, hipStream_t s);
 
 template <int NS, int NR>
@@ -831,7 +1037,10 @@ static int run_steps(mose_ctx* ctx, Case& c, int nsteps) {
   size_t iev = 0;
   for (int n = 0; n < nsteps; ++n) {
     CaseDev D0 = make_dev(ctx, c, c.P0, c.PA);
-    if (!fused || !c.dt_valid) launch_dt<NS, NR>(c, D0, s, -1);
+    if (!fused || !c.dt_valid) {
+      if (fused) D0.dtmin = c.dtnext;    // the fused step takes its dt from the slot of the next one
+      launch_dt<NS, NR>(c, D0, s, -1);
+    }
     // the fused step with dt carried over from the last stage is the same launch sequence every step: capture it
     // once and replay it (no memset node in the graph; every node is a kernel)
     const bool graph = fused && c.dt_valid && !c.timing && c.use_graph;
@@ -841,7 +1050,7 @@ static int run_steps(mose_ctx* ctx, Case& c, int nsteps) {
       continue;
     }
     if (graph) HIPCHK(ctx, hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    k_step_begin<<<1, 64, 0, s>>>(c.dt, c.dthist, c.histpos, c.hist_cap);
+    if (!fused) k_step_begin<<<1, 64, 0, s>>>(nullptr, c.dt, c.dthist, c.histpos, c.hist_cap);
     // the strang loop of Explicit_Step (Mod_Explicit.f90:155-294): one substage without chemistry; with it, half a
     // transport step (strangcoeff 1/2 in the update), Chemistry_Newstate_blk over the whole dt on the resident state,
     // the other half.  Each substage starts from the state it finds (Copy_State: P0 is the base of its stages).
@@ -853,17 +1062,11 @@ static int run_steps(mose_ctx* ctx, Case& c, int nsteps) {
         double rkc = rk[nrk - 1][irk - 1];
         const bool last = irk == nrk && istr == nstr;   // the step's last stage: next dt and the norm partials
         if (fused) {
-          int nrec = (int)c.rec.size();
-          if (nrec > 0) {
-            k_ghost<NS, NR><<<nblocks(nrec, 256), 256, 0, s>>>(D);
-            k_bcrec<NS, NR><<<nblocks(nrec, 128), 128, 0, s>>>(D);
-          }
-          if (last) k_dt_init<<<1, 64, 0, s>>>(c.dtnext);
+          launch_boundary<NS, NR>(c, D, s, irk == 1 && istr == 1);
           if (c.timing) HIPCHK(ctx, hipEventRecord(c.tev[iev++], s));
           launch_stage<NS, NR>(c, D, s, rkc, last);
           if (last) c.nparts_last = c.ntiles;
           if (c.timing) HIPCHK(ctx, hipEventRecord(c.tev[iev++], s));
-          if (last) k_dt_final<<<1, 64, 0, s>>>(c.dtnext, c.dt, nullptr, 0);
         } else {
           launch_flux<NS, NR>(c, D, s);
           if (c.sc.irs) launch_irs<NS, NR>(c, D, s);
@@ -890,6 +1093,10 @@ static int run_steps(mose_ctx* ctx, Case& c, int nsteps) {
       HIPCHK(ctx, hipGraphLaunch(c.gexec, s));
     }
     c.dt_valid = fused;
+  }
+  if (fused && nsteps > 0) {
+    k_dt_final<<<1, 64, 0, s>>>(c.dtnext, c.dt, nullptr, 0);   // between calls dt is the next step's
+    c.dead_stale = true;
   }
   HIPCHK(ctx, hipGetLastError());
   if (c.timing && iev > 0) {
@@ -929,11 +1136,7 @@ static int autotune(mose_ctx* ctx, Case& c, mose_tuning* chosen) {
     if ((TJ > 1 && dims_max[1] == 1) || (TK > 1 && dims_max[2] == 1)) continue;   // no tile across a 1-cell direction
     if (set_tiles(ctx, c, TI, TJ, TK) != MOSE_OK) continue;
     CaseDev D = make_dev(ctx, c, c.P0, c.PA);
-    int nrec = (int)c.rec.size();
-    if (nrec > 0) {
-      k_ghost<NS, NR><<<nblocks(nrec, 256), 256, 0, s>>>(D);
-      k_bcrec<NS, NR><<<nblocks(nrec, 128), 128, 0, s>>>(D);
-    }
+    launch_boundary<NS, NR>(c, D, s, false);
     launch_stage<NS, NR>(c, D, s, 1.0, false);   // warm
     HIPCHK(ctx, hipEventRecord(e0, s));
     for (int r = 0; r < 3; ++r) launch_stage<NS, NR>(c, D, s, 1.0, false);

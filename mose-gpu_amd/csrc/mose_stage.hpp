@@ -457,6 +457,12 @@ void launch_stage_tiles(const CaseDev& D, const StageArgs& A, int rs, bool visc,
   else launch_stage_shape<NS, NR, 512, 0>(D, A, rs, visc, grid, lds, s);
 }
 
+// instantiated per (NS, NR) in mose_stage.hip, one translation unit each
+extern template void launch_stage_tiles<1, 0>(const CaseDev&, const StageArgs&, int, bool, unsigned, size_t, hipStream_t);
+extern template void launch_stage_tiles<1, 1>(const CaseDev&, const StageArgs&, int, bool, unsigned, size_t, hipStream_t);
+extern template void launch_stage_tiles<4, 0>(const CaseDev&, const StageArgs&, int, bool, unsigned, size_t, hipStream_t);
+extern template void launch_stage_tiles<9, 0>(const CaseDev&, const StageArgs&, int, bool, unsigned, size_t, hipStream_t);
+
 // The performance path (mose_stage_fast.hpp), defined in its own contracted translation unit (mose_stage_fast.hip)
 // for every instantiated (NS, NR); its LDS per tile in doubles: the primitives of the tile's one-cell halo box and
 // of six slabs one cell further out, the viscous cell scalars (T alone for one species without RANS, else rho,

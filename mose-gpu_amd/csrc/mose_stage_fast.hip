@@ -1,6 +1,6 @@
 // The fused stage kernel of the performance path (MOSE_PATH_FAST, mose_stage_fast.hpp), in a translation unit
 // compiled with fused multiply-add contraction and reciprocal multiplication (the library's Makefile gives the flags).
-// The parity kernels (mose_capi.hip) keep the reference's roundings.
+// The parity kernels (mose_stage.hip) keep the reference's roundings.  One object per (MOSE_NS, MOSE_NR).
 #include <hip/hip_runtime.h>
 
 #include "mose_stage_fast.hpp"
@@ -37,9 +37,7 @@ void launch_stage_fast(const CaseDev& D, const StageArgs& A, int rs, bool visc, 
   launch_fast_shape<NS, NR, 512, 0>(D, A, rs, visc, grid, lds, s);
 }
 
-template void launch_stage_fast<1, 0>(const CaseDev&, const StageArgs&, int, bool, unsigned, size_t, hipStream_t);
-template void launch_stage_fast<1, 1>(const CaseDev&, const StageArgs&, int, bool, unsigned, size_t, hipStream_t);
-template void launch_stage_fast<4, 0>(const CaseDev&, const StageArgs&, int, bool, unsigned, size_t, hipStream_t);
-template void launch_stage_fast<9, 0>(const CaseDev&, const StageArgs&, int, bool, unsigned, size_t, hipStream_t);
+template void launch_stage_fast<MOSE_NS, MOSE_NR>(const CaseDev&, const StageArgs&, int, bool, unsigned, size_t,
+                                                  hipStream_t);
 
 }  // namespace mose
