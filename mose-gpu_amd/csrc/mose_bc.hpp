@@ -178,14 +178,16 @@ __device__ __forceinline__ void bc_euler(const CaseDev& C, const BcPlan& p, cons
     }
     const double D12 = Dl1 + Dl2, D23 = Dl2 + Dl3, D34 = Dl3 + Dl4;
     double L[NP], R[NP];
+    with_limiter(C.lim, [&](auto lim) {
 #pragma unroll
-    for (int s = 0; s < NP; ++s) {
-      const double a1 = modfm ? q2[s] : qi[s], a2 = modfm ? q1[s] : qc[s], a3 = modfm ? qc[s] : q1[s],
-                   a4 = modfm ? qi[s] : q2[s];
-      const double d21 = (a2 - a1) / D12, d32 = (a3 - a2) / D23, d43 = (a4 - a3) / D34;
-      L[s] = a2 + 1.0 * limiter(C.lim, d32, d21) * Dl2;
-      R[s] = a3 - 1.0 * limiter(C.lim, d43, d32) * Dl3;
-    }
+      for (int s = 0; s < NP; ++s) {
+        const double a1 = modfm ? q2[s] : qi[s], a2 = modfm ? q1[s] : qc[s], a3 = modfm ? qc[s] : q1[s],
+                     a4 = modfm ? qi[s] : q2[s];
+        const double d21 = (a2 - a1) / D12, d32 = (a3 - a2) / D23, d43 = (a4 - a3) / D34;
+        L[s] = a2 + 1.0 * limiter(lim.id, d32, d21) * Dl2;
+        R[s] = a3 - 1.0 * limiter(lim.id, d43, d32) * Dl3;
+      }
+    });
     const double rL = rho_sum<NS>(L), RL = f_Rtot<NS>(T, L), rR = rho_sum<NS>(R), RR = f_Rtot<NS>(T, R);
     const double aL = f_ss<NS>(T, L, L[V::np], rL, RL), aR = f_ss<NS>(T, R, R[V::np], rR, RR);
     const F5 F = riemann<NS>(T, C.rs, C.mco, false, L, L[V::nu], L[V::nv], L[V::nw], L[V::np], aL, rL, R, R[V::nu],

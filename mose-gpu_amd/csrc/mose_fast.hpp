@@ -5,7 +5,6 @@
 // relative L-infinity <= 1e-12 on this path too.
 //
 // What changes:
-//   half_slope_fast  the van Leer and van Albada limiters with one division in place of two (below)
 //   conv_face_fast  LMRoe (riemann_open_body.inc:965-1090) and its Roe averages (:679-726) evaluated once per face:
 //                   one reciprocal per side density, the face's species fractions, enthalpies and mixture gas
 //                   constant shared by the averages and the physical fluxes (the reference recomputes them in
@@ -20,30 +19,6 @@
 #include "mose_physics.hpp"
 
 namespace mose {
-
-// The limiters of Lib_Limiters.f90:65-97 with one division: the ratio forms phi(ru) x, ru = y / (x + 1e-30), of van
-// Leer and van Albada multiplied through by the denominator's |x'| or x'^2 (x' = x + 1e-30):
-//   van Leer    (ru + |ru|) / (1 + |ru|) x = (y sgn(x') + |y|) / (|x'| + |y|) x
-//   van Albada  (ru^2 + ru) / (1 + ru^2) x = (y^2 + y x') / (x'^2 + y^2) x
-// minmod has no division; MC and superbee keep their one division.
-__device__ __forceinline__ double limiter_fast(int lim, double x, double y) {
-  if (lim == 2) {
-    const double xp = x + 1e-30;
-    return ((xp < 0.0 ? -y : y) + fabs(y)) / (fabs(xp) + fabs(y)) * x;
-  }
-  if (lim == 3) {
-    const double xp = x + 1e-30;
-    return (y * y + y * xp) / (xp * xp + y * y) * x;
-  }
-  return limiter(lim, x, y);
-}
-
-// half_slope (mose_physics.hpp) with limiter_fast
-__device__ __forceinline__ double half_slope_fast(int lim, double qm, double q0, double qp, double idlm, double idlp,
-                                                  double hdl) {
-  const double s0 = (q0 - qm) * idlm, s1 = (qp - q0) * idlp;
-  return limiter_fast(lim, s1, s0) * hdl;
-}
 
 template <int NS, int NR>
 __device__ __forceinline__ void conv_face_lmroe_fast(const mose_dtab& T, double mco, double* L, double* R, double nx,

@@ -155,6 +155,25 @@ __device__ __forceinline__ double limiter(int lim, double x, double y) {
   }
 }
 
+// f(LimId<limiter>{}) with the case's limiter as a compile-time constant: one uniform branch around all the slopes of a
+// face or cell.  With the run-time limiter inside the loop over the variables each of its 5 to 10 evaluations is a
+// basic block of its own, so their loads and their division chains ran one after another; inside f they overlap.
+// Shock tube of 1000 cells, 100 steps: 6.88 -> 6.61 ms; 101 x 97 x 89 Taylor-Green, 10 parity steps: 12.84 -> 12.26 ms;
+// 64 x 64 Riemann problem on the performance path, 40 steps: 2.59 -> 2.45 ms.
+template <int L>
+struct LimId { static constexpr int id = L; };
+template <class F>
+__device__ __forceinline__ void with_limiter(int lim, F&& f) {
+  switch (lim) {
+    case 1: f(LimId<1>{}); break;
+    case 2: f(LimId<2>{}); break;
+    case 3: f(LimId<3>{}); break;
+    case 4: f(LimId<4>{}); break;
+    case 5: f(LimId<5>{}); break;
+    default: f(LimId<6>{}); break;
+  }
+}
+
 // ---------------------------------------------------------------------------------------------------------
 // one side of a face: species densities + u v w p, and its mixture rho / R / sound speed
 // ---------------------------------------------------------------------------------------------------------

@@ -215,10 +215,13 @@ __device__ __forceinline__ void stage_tile(const CaseDev& C, const StageArgs& A,
     const double* dlp = C.dl + (int64_t)d * NC;
     double dm = dlp[c0 - st], d0 = dlp[c0], dp = dlp[c0 + st];
     double idm = 1.0 / (0.5 * (dm + d0)), idp = 1.0 / (0.5 * (d0 + dp)), hd = 0.5 * d0;
+    double qm[NP], q0[NP], qp[NP];
 #pragma unroll
-    for (int s = 0; s < NP; ++s) {
-      Hs[s * G.nhs + q] = half_slope(C.lim, P[s * NC + c0 - st], P[s * NC + c0], P[s * NC + c0 + st], idm, idp, hd);
-    }
+    for (int s = 0; s < NP; ++s) { qm[s] = P[s * NC + c0 - st]; q0[s] = P[s * NC + c0]; qp[s] = P[s * NC + c0 + st]; }
+    with_limiter(C.lim, [&](auto lim) {
+#pragma unroll
+      for (int s = 0; s < NP; ++s) Hs[s * G.nhs + q] = half_slope(lim.id, qm[s], q0[s], qp[s], idm, idp, hd);
+    });
   }
   __syncthreads();
 

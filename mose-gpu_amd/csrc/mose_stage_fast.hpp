@@ -64,7 +64,11 @@ __device__ __forceinline__ double rcp_nr(double x) {
   return fma(e, r, r);
 }
 
-// The limiters of Lib_Limiters.f90:65-97 in their one-division forms (limiter_fast) with the reciprocal above
+// The limiters of Lib_Limiters.f90:65-97 with one reciprocal: the ratio forms phi(ru) x, ru = y / (x + 1e-30), of van
+// Leer and van Albada multiplied through by the denominator's |x'| or x'^2 (x' = x + 1e-30):
+//   van Leer    (ru + |ru|) / (1 + |ru|) x = (y sgn(x') + |y|) / (|x'| + |y|) x
+//   van Albada  (ru^2 + ru) / (1 + ru^2) x = (y^2 + y x') / (x'^2 + y^2) x
+// minmod has no division; MC and superbee keep their one division.
 __device__ __forceinline__ double limiter_nr(int lim, double x, double y) {
   if (lim == 2) {
     const double xp = x + 1e-30;
@@ -423,13 +427,15 @@ __device__ __forceinline__ void stage_tile_fast(const CaseDev& C, const StageArg
     const double i0 = rcp_nr(0.5 * (dLL + dL)), i1 = rcp_nr(0.5 * (dL + dR)), i2 = rcp_nr(0.5 * (dR + dRR));
     const double hL = 0.5 * dL, hR = 0.5 * dR;
     double L[NP], R[NP], res[NP];
+    with_limiter(C.lim, [&](auto lim) {
 #pragma unroll
-    for (int s = 0; s < NP; ++s) {
-      const double* q = Pl + s * NX;
-      const double qLL = q[kLL], qL = q[kL], qR = q[kR], qRR = q[kRR];
-      L[s] = qL + limiter_nr(C.lim, (qR - qL) * i1, (qL - qLL) * i0) * hL;
-      R[s] = qR - limiter_nr(C.lim, (qRR - qR) * i2, (qR - qL) * i1) * hR;
-    }
+      for (int s = 0; s < NP; ++s) {
+        const double* q = Pl + s * NX;
+        const double qLL = q[kLL], qL = q[kL], qR = q[kR], qRR = q[kRR];
+        L[s] = qL + limiter_nr(lim.id, (qR - qL) * i1, (qL - qLL) * i0) * hL;
+        R[s] = qR - limiter_nr(lim.id, (qRR - qR) * i2, (qR - qL) * i1) * hR;
+      }
+    });
     conv_face_fast<NS, NR, RS>(T, C.rs, C.mco, L, R, fnx, fny, fnz, fa, res);
 #pragma unroll
     for (int s = 0; s < NP; ++s) Fb[s * NF + f] = res[s];
