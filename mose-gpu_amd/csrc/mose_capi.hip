@@ -66,6 +66,7 @@ struct Case {
   int TI = 32, TJ = 4, TK = 2;
   Tile* dtiles = nullptr;
   int ntiles = 0, tiles_cap = 0;
+  int flat = 0, flat_bs = 0;         // the stage runs mose_flat.hpp (flat_dims), with this many threads a tile
   unsigned long long* dtnext = nullptr;
   bool dt_valid = false;
   // the planned boundary kernel of the fused paths (k_bc) for the records that act in every stage; ndead others have
@@ -117,6 +118,7 @@ struct Case {
 struct mose_ctx {
   int device = 0;
   int max_lds = 65536;       // dynamic LDS a workgroup may take on this device
+  int cus = 0;               // its compute units
   hipStream_t stream = nullptr;
   int nsc = 0;
   bool viscous_tables = false;
@@ -203,6 +205,7 @@ extern "C" int mose_ctx_create(int device, const mose_tables* t, mose_ctx** out)
     int v = 0;
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, device) == hipSuccess && v > 0)
       ctx->max_lds = v;
+    HIPCHK(ctx.get(), hipDeviceGetAttribute(&ctx->cus, hipDeviceAttributeMultiprocessorCount, device));
   }
   size_t n = (size_t)t->nsc * MOSE_NTAB;
   HIPCHK(ctx.get(), hipMalloc(&ctx->dcp, 4 * n * sizeof(double)));
@@ -681,15 +684,50 @@ static Case* get_case(mose_ctx* ctx, int id) {
   ((sc).nsc == 9 ? F<9, 0>(__VA_ARGS__) : (sc).nsc == 4 ? F<4, 0>(__VA_ARGS__)                          \
                                         : (sc).nrans == 0 ? F<1, 0>(__VA_ARGS__) : F<1, 1>(__VA_ARGS__))
 
+// The device code of a path's stage kernels, asked for ahead of the first step (stage_kernel_parity in mose_stage.hpp)
+template <int NS, int NR>
+static int load_stage(mose_ctx* ctx, int path) {
+  hipFuncAttributes a;
+  HIPCHK(ctx, hipFuncGetAttributes(&a, path == MOSE_PATH_FAST ? stage_kernel_fast<NS, NR>() : stage_kernel_parity<NS, NR>()));
+  return MOSE_OK;
+}
+
 static size_t stage_lds_(int nprim, bool visc, int TI, int TJ, int TK);
 // static LDS of the stage kernel beside its dynamic part (the workgroup reductions of dt and of the residual norm)
 static constexpr size_t kStaticLds = 2048;
+// The stage of a case runs mose_flat.hpp (0: the general kernels, 1: rows, 2: planes) where no block is more than one cell
+// thick in k and the tile is a plane too, for one species without RANS, inviscid; a tile of 512 cells has more cells than
+// that kernel takes threads.
+static int flat_dims(const Case& c, int TI, int TJ, int TK) {
+  if (c.sc.viscous || c.sc.nsc != 1 || c.sc.nrans != 0 || TK != 1 || TI * TJ > 256) return 0;
+  bool two = false;
+  for (auto& B : c.blk) {
+    if (B.n3 != 1) return 0;
+    two = two || B.n2 > 1;
+  }
+  return 1 + two;
+}
+
+static int64_t tile_count(const Case& c, int TI, int TJ, int TK) {
+  int64_t n = 0;
+  for (auto& B : c.blk) n += (int64_t)((B.n1 + TI - 1) / TI) * ((B.n2 + TJ - 1) / TJ) * ((B.n3 + TK - 1) / TK);
+  return n;
+}
+
 // the first tile of the preference list that fits the device's LDS and does not straddle a one-cell direction
 static void choose_default_tile(mose_ctx* ctx, Case& c) {
   static const int pref[][3] = {{8, 8, 4}, {16, 4, 4}, {32, 4, 2}, {16, 8, 2}, {32, 8, 1}, {64, 4, 1}, {16, 16, 1},
                                 {128, 2, 1}, {256, 1, 1}};
   int mx[3] = {0, 0, 0};
   for (auto& B : c.blk) { mx[0] = std::max(mx[0], B.n1); mx[1] = std::max(mx[1], B.n2); mx[2] = std::max(mx[2], B.n3); }
+  // planes and rows: tiles of 128 cells while flat_threads gives them a thread per face
+  if (const int dims = flat_dims(c, 16, 8, 1)) {
+    const int TI = dims == 2 ? 16 : 128, TJ = dims == 2 ? 8 : 1;
+    if (flat_threads(TI, TJ, dims == 2, tile_count(c, TI, TJ, 1), ctx->cus) > TI * TJ) {
+      c.TI = TI; c.TJ = TJ; c.TK = 1;
+      return;
+    }
+  }
   for (auto& t : pref) {
     if ((t[1] > 1 && mx[1] == 1) || (t[2] > 1 && mx[2] == 1)) continue;
     if (stage_lds_(c.nprim, c.sc.viscous != 0, t[0], t[1], t[2]) + kStaticLds > (size_t)ctx->max_lds) continue;
@@ -744,14 +782,16 @@ extern "C" int mose_case_create(mose_ctx* ctx, const mose_scheme* sc, int nb, co
   }
   HIPCHK(ctx, hipStreamSynchronize(s));
   rc = plan_boundary(ctx, *c, s);
-  if (rc == MOSE_OK) rc = ensure_rpart(ctx, *c, plain_parts(*c));
+  if (rc == MOSE_OK && c->path != MOSE_PATH_PLAIN) rc = MOSE_DISPATCH(c->sc, load_stage, ctx, c->path);
+  choose_default_tile(ctx, *c);
+  // the norm partials of either path: growing them in the first step is a free (5 ms)
+  if (rc == MOSE_OK) rc = ensure_rpart(ctx, *c, std::max(plain_parts(*c), tile_count(*c, c->TI, c->TJ, c->TK)));
   if (rc != MOSE_OK) { case_free(c.get()); return rc; }
   c->valid = true;
   {
     const char* e = std::getenv("MOSE_NO_GRAPH");
     if (e && e[0] == '1') c->use_graph = false;
   }
-  choose_default_tile(ctx, *c);
   ctx->cases.push_back(std::move(c));
   *case_id = (int)ctx->cases.size() - 1;
   return MOSE_OK;
@@ -985,6 +1025,8 @@ static int set_tiles(mose_ctx* ctx, Case& c, int TI, int TJ, int TK) {
   HIPCHK(ctx, hipStreamSynchronize(c.stream));
   c.ntiles = (int)t.size();
   c.TI = TI; c.TJ = TJ; c.TK = TK;
+  c.flat = flat_dims(c, TI, TJ, TK);
+  if (c.flat) c.flat_bs = flat_threads(TI, TJ, c.flat == 2, c.ntiles, ctx->cus);
   drop_graph(c);
   return ensure_rpart(ctx, c, c.ntiles);
 }
@@ -1006,6 +1048,12 @@ static void launch_stage(Case& c, const CaseDev& D, hipStream_t s, double rkc, b
   A.last = last ? 1 : 0; A.rkc = rkc; A.dtnext = c.dtnext; A.rpart = c.rpart;
   size_t lds = stage_lds(c, c.TI, c.TJ, c.TK);
   unsigned grid = (unsigned)(((c.ntiles + 7) / 8) * 8);
+  if constexpr (NS == 1 && NR == 0) {
+    if (c.flat) {
+      (c.path == MOSE_PATH_FAST ? launch_flat_fast : launch_flat_parity)(D, A, c.sc.riemann, c.flat == 2, c.flat_bs, grid, s);
+      return;
+    }
+  }
   if (c.path == MOSE_PATH_FAST) launch_stage_fast<NS, NR>(D, A, c.sc.riemann, c.sc.viscous != 0, grid, lds, s);
   else launch_stage_tiles<NS, NR>(D, A, c.sc.riemann, c.sc.viscous != 0, grid, lds, s);
 }
@@ -1119,7 +1167,7 @@ static int autotune(mose_ctx* ctx, Case& c, mose_tuning* chosen) {
   // buffer PA, the state P0 untouched) a few times, the fastest is kept
   static const int cand[][3] = {{32, 4, 2}, {64, 2, 2}, {16, 4, 4}, {16, 8, 2}, {8, 8, 4}, {64, 4, 1}, {32, 8, 1},
                                 {128, 2, 1}, {256, 1, 1}, {8, 8, 8}, {16, 8, 4}, {16, 4, 8}, {32, 4, 4}, {16, 16, 2},
-                                {32, 16, 1}, {64, 8, 1}, {8, 4, 4}, {16, 4, 2}, {16, 8, 1}};
+                                {32, 16, 1}, {64, 8, 1}, {8, 4, 4}, {16, 4, 2}, {16, 8, 1}, {128, 1, 1}};
   hipStream_t s = c.stream;
   hipEvent_t e0, e1;
   HIPCHK(ctx, hipEventCreate(&e0));
@@ -1180,6 +1228,8 @@ extern "C" int mose_case_tune(mose_ctx* ctx, int id, const mose_tuning* t, mose_
   drop_graph(*c);
   if (chosen) *chosen = *t;
   if (c->path == MOSE_PATH_FUSED || c->path == MOSE_PATH_FAST) {
+    const int rc = MOSE_DISPATCH(c->sc, load_stage, ctx, c->path);
+    if (rc != MOSE_OK) return rc;
     if (t->ti == 0 && t->tj == 0 && t->tk == 0)
       return MOSE_DISPATCH(c->sc, autotune, ctx, *c, chosen);
     return set_tiles(ctx, *c, t->ti, t->tj, t->tk);

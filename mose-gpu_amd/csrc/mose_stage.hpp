@@ -474,6 +474,30 @@ template <int NS, int NR>
 void launch_stage_fast(const CaseDev& D, const StageArgs& A, int rs, bool visc, unsigned grid, size_t lds,
                        hipStream_t s);
 
+// A kernel of each of those translation units: the runtime loads a unit's code when it first meets one of its kernels
+// (3 ms), and the host asks for it when a case is made or tuned rather than in its first step.
+template <int NS, int NR>
+const void* stage_kernel_parity();
+template <int NS, int NR>
+const void* stage_kernel_fast();
+
+// The planes of mose_flat.hpp: the threads of a workgroup and the LDS doubles of a TI x TJ tile (`two`: with j-faces); the
+// launches of both paths are defined in mose_stage_fast.hip and mose_stage.hip.
+// One thread per cell; one per face (320 at most: tiles of 128 cells, or 256 in one dimension) while every tile is resident
+// at once, at three of these workgroups on a CU: a thread's chain is then one face long.
+// A stage of 128-cell tiles with a thread per face and per cell: 32 tiles 16 and 21 us, 512 tiles 21 and 26 us, 1152 tiles
+// 39 and 36 us, 2048 tiles 59 and 48 us.
+constexpr int FLAT_THREADS = 320;
+constexpr int flat_threads(int TI, int TJ, bool two, int64_t ntiles, int cus) {
+  const int wide = (two ? 2 : 1) * TI * TJ + ((TJ + (two ? TI : 0) + 63) & ~63);
+  return wide <= FLAT_THREADS && ntiles <= 3 * cus ? wide : TI * TJ;
+}
+constexpr size_t flat_lds_doubles(int TI, int TJ, bool two) {
+  return 5 * ((size_t)TI * TJ + 4 * TJ + (two ? 4 * TI : 0) + (size_t)(TI + 1) * TJ + (two ? (size_t)TI * (TJ + 1) : 0));
+}
+void launch_flat_parity(const CaseDev& D, const StageArgs& A, int rs, bool two, int threads, unsigned grid, hipStream_t s);
+void launch_flat_fast(const CaseDev& D, const StageArgs& A, int rs, bool two, int threads, unsigned grid, hipStream_t s);
+
 inline size_t fast_lds_doubles(int ns, int nr, int nprim, bool visc, int TI, int TJ, int TK) {
   const size_t nbox = (size_t)(TI + 2) * (TJ + 2) * (TK + 2);
   const size_t next = nbox + 2 * ((size_t)TJ * TK + (size_t)TI * TK + (size_t)TI * TJ);

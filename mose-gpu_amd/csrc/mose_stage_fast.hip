@@ -3,7 +3,7 @@
 // The parity kernels (mose_stage.hip) keep the reference's roundings.  One object per (MOSE_NS, MOSE_NR).
 #include <hip/hip_runtime.h>
 
-#include "mose_stage_fast.hpp"
+#include "mose_flat.hpp"
 
 namespace mose {
 
@@ -39,5 +39,17 @@ void launch_stage_fast(const CaseDev& D, const StageArgs& A, int rs, bool visc, 
 
 template void launch_stage_fast<MOSE_NS, MOSE_NR>(const CaseDev&, const StageArgs&, int, bool, unsigned, size_t,
                                                   hipStream_t);
+
+template <int NS, int NR>
+const void* stage_kernel_fast() {
+  return (const void*)k_stage_fast<NS, NR, false, MOSE_RS_HLLC, 256, 0>;
+}
+template const void* stage_kernel_fast<MOSE_NS, MOSE_NR>();
+
+#if MOSE_NS == 1 && MOSE_NR == 0
+void launch_flat_fast(const CaseDev& D, const StageArgs& A, int rs, bool two, int threads, unsigned grid, hipStream_t s) {
+  launch_flat<true>(D, A, rs, two, threads, grid, s);
+}
+#endif
 
 }  // namespace mose

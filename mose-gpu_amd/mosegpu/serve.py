@@ -94,15 +94,19 @@ class ServeStats:
 
 def serve_tile(case, path: int):
     """The stage tile of a served case, by rule instead of the autotuner (which would time candidate tiles on every
-    admitted case while the others wait): 8 x 8 x 4 for 3D blocks, 16 x 8 x 1 for 2D ones (a 128-cell tile: a 256-cell
-    2D tile's LDS, most of it for the unused one-cell direction, leaves one workgroup per CU; on a 1024^2 Riemann
-    case a stage takes 0.25 ms against 0.33 ms with 32 x 8 x 1)."""
+    admitted case while the others wait): 8 x 8 x 4 for 3D blocks; 2D ones 16 x 8 x 1, 32 x 8 x 1 from about 100,000 cells
+    on if inviscid (a stage of a 256^2 Riemann case takes 21 against 23 us, of a 1024^2 one 152 against 135 us; a viscous
+    256-cell tile's LDS, most of it for the unused one-cell direction, leaves one workgroup per CU); 1D ones 128 x 1 x 1,
+    256 x 1 x 1 if viscous (1,000 inviscid cells: 16 against 19 us, 200,000 cells: 73 against 72 us)."""
     if path == PATH_PLAIN:
         return (0, 0, 0)
     n1, n2, n3 = case.layout.dims[0]
-    if n3 == 1:
-        return (16, 8, 1) if n2 > 1 else (256, 1, 1)
-    return (8, 8, 4)
+    if n3 > 1:
+        return (8, 8, 4)
+    large, euler = n1 * n2 > 768 * 128, not case.scheme.viscous
+    if n2 > 1:
+        return (32, 8, 1) if large and euler else (16, 8, 1)
+    return (128, 1, 1) if euler else (256, 1, 1)
 
 
 def serve(reqs: list[Request], budget_bytes: int | None = None, quantum: int = 10, path: int = PATH_FUSED,
