@@ -468,7 +468,7 @@ extern template void launch_stage_tiles<9, 0>(const CaseDev&, const StageArgs&, 
 
 // The performance path (mose_stage_fast.hpp), defined in its own contracted translation unit (mose_stage_fast.hip)
 // for every instantiated (NS, NR); its LDS per tile in doubles: the primitives of the tile's one-cell halo box and
-// of six slabs one cell further out, the viscous cell scalars (T alone for one species without RANS, else rho,
+// of six slabs one cell further out, the viscous cell scalars (T, with RANS 1/rho, for one species, else rho,
 // 1/rho, T), the face slots.
 template <int NS, int NR>
 void launch_stage_fast(const CaseDev& D, const StageArgs& A, int rs, bool visc, unsigned grid, size_t lds,
@@ -502,7 +502,7 @@ inline size_t fast_lds_doubles(int ns, int nr, int nprim, bool visc, int TI, int
   const size_t nbox = (size_t)(TI + 2) * (TJ + 2) * (TK + 2);
   const size_t next = nbox + 2 * ((size_t)TJ * TK + (size_t)TI * TK + (size_t)TI * TJ);
   const size_t nslot = (size_t)(TI + 1) * TJ * TK + (size_t)TI * (TJ + 1) * TK + (size_t)TI * TJ * (TK + 1);
-  const size_t ncc = visc ? ((ns == 1 && nr == 0) ? 1 : 3) : 0;
+  const size_t ncc = visc ? (ns == 1 ? (nr == 0 ? 1 : 2) : 3) : 0;
   // one species without RANS on 8 x 8 x 4 tiles: 128 doubles for the staged cell metrics of the viscous faces
   const size_t mst = (visc && ns == 1 && nr == 0 && TI == 8 && TJ == 8 && TK == 4) ? 128 : 0;
   return (size_t)nprim * next + ncc * nbox + mst + (size_t)nprim * nslot;
