@@ -57,8 +57,8 @@ static __global__ void __launch_bounds__(64) k_bc_geometry(CaseDev C, const BcPl
   const BcPlan p = plan[t];
   const int d = (p.meta >> BCP_DIR) & 3;
   const double* fm = d == 0 ? C.fm1 : (d == 1 ? C.fm2 : C.fm3);
-  const int64_t NF = d == 0 ? C.NF1 : (d == 1 ? C.NF2 : C.NF3), N = n, c = p.c, in = bcp_in(C, p);
-  for (int q = 0; q < 4; ++q) geo[q * N + t] = fm[q * NF + p.fg];
+  const int64_t N = n, c = p.c, in = bcp_in(C, p);
+  for (int q = 0; q < 4; ++q) geo[q * N + t] = fm[4 * (int64_t)p.fg + q];
   const double* dlp = C.dl + (int64_t)d * C.NC;
   geo[BCG_DL * N + t] = dlp[c - 2 * in];
   geo[(BCG_DL + 1) * N + t] = dlp[c - in];
@@ -66,7 +66,7 @@ static __global__ void __launch_bounds__(64) k_bc_geometry(CaseDev C, const BcPl
   const mose_blk B = C.blk[p.b];
   geo[(BCG_DL + 3) * N + t] = dlp[(d == 0 ? B.n1 : (d == 1 ? B.n2 : B.n3)) > 1 ? c + in : c];
   if (!C.visc) return;
-  for (int q = 0; q < 9; ++q) geo[(BCG_M + q) * N + t] = 0.5 * (C.m[(int64_t)q * C.NC + c] + C.m[(int64_t)q * C.NC + c - in]);
+  for (int q = 0; q < 9; ++q) geo[(BCG_M + q) * N + t] = 0.5 * (C.m[9 * c + q] + C.m[9 * (c - in) + q]);
 }
 
 // The part of a step's start that the first stage's boundary kernel does (one thread): dt and its history from the

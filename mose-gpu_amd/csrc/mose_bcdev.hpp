@@ -92,7 +92,7 @@ __device__ __forceinline__ void bc_wall_visc(const mose_dtab& T, const double* P
 #pragma unroll
   for (int a = 0; a < 3; ++a)
 #pragma unroll
-    for (int c = 0; c < 3; ++c) M[a][c] = m[(int64_t)(a + 3 * c) * NC + rc.c];
+    for (int c = 0; c < 3; ++c) M[a][c] = m[9 * (int64_t)rc.c + a + 3 * c];
   double rho = rho_sum<NS>(Pb), Rg = f_Rtot<NS>(T, Pb);
   double Tk = Pb[V::np] / (rho * Rg), mil, kl;
   if (typ == MOSE_BC_WALL_ADIABATIC) {
@@ -149,7 +149,7 @@ __device__ __forceinline__ void bc_sym_visc_n(const mose_dtab& T, const double* 
 #pragma unroll
   for (int x = 0; x < 3; ++x)
 #pragma unroll
-    for (int y = 0; y < 3; ++y) M[x][y] = m[(int64_t)(x + 3 * y) * NC + rc.c];
+    for (int y = 0; y < 3; ++y) M[x][y] = m[9 * (int64_t)rc.c + x + 3 * y];
   double rho = rho_sum<NS>(Pb), Rg = f_Rtot<NS>(T, Pb);
   double Tk = Pb[V::np] / (rho * Rg), mil, kl;
   int Ti = ftrunc(Tk);
@@ -455,7 +455,7 @@ __device__ __forceinline__ double sa_source(const double* P, int64_t NC, const d
 #pragma unroll
   for (int a = 0; a < 3; ++a)
 #pragma unroll
-    for (int c = 0; c < 3; ++c) M[a][c] = m[(int64_t)(a + 3 * c) * NC + c0];
+    for (int c = 0; c < 3; ++c) M[a][c] = m[9 * c0 + a + 3 * c];
   double ntv[6], sum[6];
 #pragma unroll
   for (int q = 0; q < 6; ++q) {

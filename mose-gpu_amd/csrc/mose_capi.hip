@@ -758,13 +758,22 @@ extern "C" int mose_case_create(mose_ctx* ctx, const mose_scheme* sc, int nb, co
   HIPCHK(ctx, hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));   // default priority
   hipStream_t s = c->stream;
   HIPCHK(ctx, hipMemcpyAsync(c->dl, dl, 3 * (size_t)c->NC * d, hipMemcpyHostToDevice, s));
-  HIPCHK(ctx, hipMemcpyAsync(c->m, m, 9 * (size_t)c->NC * d, hipMemcpyHostToDevice, s));
+  // metrics and face geometry arrive component by component and are kept cell by cell and face by face; the state buffers
+  // (15 components or more of the arena's cells) hold them on the way
+  auto packed = [&](double* dst, const double* src, int k, int64_t n) -> hipError_t {
+    if (n == 0) return hipSuccess;
+    hipError_t e = hipMemcpyAsync(c->P0, src, (size_t)k * n * d, hipMemcpyHostToDevice, s);
+    if (e != hipSuccess) return e;
+    k_pack<<<nblocks(n, 256), 256, 0, s>>>(c->P0, dst, n, k);
+    return hipGetLastError();
+  };
+  HIPCHK(ctx, packed(c->m, m, 9, c->NC));
   HIPCHK(ctx, hipMemcpyAsync(c->vol, vol, (size_t)c->NC * d, hipMemcpyHostToDevice, s));
   if (yn) HIPCHK(ctx, hipMemcpyAsync(c->yn, yn, (size_t)c->NC * d, hipMemcpyHostToDevice, s));
   else HIPCHK(ctx, hipMemsetAsync(c->yn, 0, (size_t)c->NC * d, s));
-  HIPCHK(ctx, hipMemcpyAsync(c->fm1, fm1, 4 * (size_t)c->NF1 * d, hipMemcpyHostToDevice, s));
-  HIPCHK(ctx, hipMemcpyAsync(c->fm2, fm2, 4 * (size_t)c->NF2 * d, hipMemcpyHostToDevice, s));
-  HIPCHK(ctx, hipMemcpyAsync(c->fm3, fm3, 4 * (size_t)c->NF3 * d, hipMemcpyHostToDevice, s));
+  HIPCHK(ctx, packed(c->fm1, fm1, 4, c->NF1));
+  HIPCHK(ctx, packed(c->fm2, fm2, 4, c->NF2));
+  HIPCHK(ctx, packed(c->fm3, fm3, 4, c->NF3));
   HIPCHK(ctx, hipMemcpyAsync(c->dblk, c->blk.data(), c->blk.size() * sizeof(mose_blk), hipMemcpyHostToDevice, s));
   if (!c->rec.empty())
     HIPCHK(ctx, hipMemcpyAsync(c->drec, c->rec.data(), c->rec.size() * sizeof(mose_bc_record), hipMemcpyHostToDevice, s));
@@ -840,7 +849,7 @@ extern "C" int mose_state_download(mose_ctx* ctx, int id, double* P) {
 static CaseDev make_dev(mose_ctx* ctx, Case& c, const double* Pin, double* Pout) {
   CaseDev D{};
   D.Pin = Pin; D.Pout = Pout; D.PO = c.P0; D.Pg = const_cast<double*>(Pin);
-  D.NC = c.NC; D.NF1 = c.NF1; D.NF2 = c.NF2; D.NF3 = c.NF3;
+  D.NC = c.NC;
   D.dl = c.dl; D.m = c.m; D.vol = c.vol; D.yn = c.yn; D.fm1 = c.fm1; D.fm2 = c.fm2; D.fm3 = c.fm3;
   for (int q = 0; q < 3; ++q) { D.Fc[q] = c.Fc[q]; D.Fd[q] = c.Fd[q]; D.NFI[q] = c.NFI[q]; }
   D.binc = c.binc; D.NBP = std::max<int64_t>(c.NBP, 1);

@@ -84,10 +84,9 @@ __global__ void __launch_bounds__(WIDE ? FLAT_THREADS : 256, (!FAST && RS == MOS
       const double* dlp = C.dl + d * NC + row(B, i, j, 1);
       const int64_t st = d ? sj : 1;
       dLL = dlp[-2 * st]; dL = dlp[-st]; dR = dlp[0]; dRR = dlp[st];
-      const int64_t NFg = d ? C.NF2 : C.NF1;
-      const double* fm = d ? C.fm2 + B.f2off + (i - 1) + (int64_t)B.n1 * (j - 1)
-                           : C.fm1 + B.f1off + (i - 1) + (int64_t)(B.n1 + 1) * (j - 1);
-      nx = fm[0]; ny = fm[NFg]; nz = fm[2 * NFg]; area = fm[3 * NFg];
+      const double* fm = d ? C.fm2 + 4 * (B.f2off + (i - 1) + (int64_t)B.n1 * (j - 1))
+                           : C.fm1 + 4 * (B.f1off + (i - 1) + (int64_t)(B.n1 + 1) * (j - 1));
+      nx = fm[0]; ny = fm[1]; nz = fm[2]; area = fm[3];
     }
     if (r0 == 0) __syncthreads();             // the LDS stencil, with the first face's geometry in flight
     if (face) {

@@ -97,16 +97,15 @@ __device__ __forceinline__ void visc_face(const CaseDev& C, const mose_blk& B, c
   for (int s = 0; s < NP; ++s) Pf[s] = 0.5 * (Pc[s * NCa + k1] + Pc[s * NCa + k2]);
   const FaceThermo ft = face_thermo<NS>(T, Pf, Pf[V::np], C.vc.prl);
   const double* fm = D == 0 ? C.fm1 : (D == 1 ? C.fm2 : C.fm3);
-  const int64_t NFg = D == 0 ? C.NF1 : (D == 1 ? C.NF2 : C.NF3);
   const int64_t fg = D == 0 ? B.f1off + i + (int64_t)(B.n1 + 1) * ((j - 1) + (int64_t)B.n2 * (k - 1))
                    : D == 1 ? B.f2off + (i - 1) + (int64_t)B.n1 * (j + (int64_t)(B.n2 + 1) * (k - 1))
                             : B.f3off + (i - 1) + (int64_t)B.n1 * ((j - 1) + (int64_t)B.n2 * k);
-  const double nx = fm[fg], ny = fm[NFg + fg], nz = fm[2 * NFg + fg], area = fm[3 * NFg + fg];
+  const double nx = fm[4 * fg], ny = fm[4 * fg + 1], nz = fm[4 * fg + 2], area = fm[4 * fg + 3];
   double Mav[3][3];
 #pragma unroll
   for (int x = 0; x < 3; ++x)
 #pragma unroll
-    for (int y = 0; y < 3; ++y) Mav[x][y] = 0.5 * (C.m[(int64_t)(x + 3 * y) * NC + c0] + C.m[(int64_t)(x + 3 * y) * NC + c1]);
+    for (int y = 0; y < 3; ++y) Mav[x][y] = 0.5 * (C.m[9 * c0 + x + 3 * y] + C.m[9 * c1 + x + 3 * y]);
   const double drho = ft.rho, dmil = ft.mil;
   const int Ti = ftrunc(ft.T);
   const double Tdf = ft.T - Ti;
@@ -249,11 +248,10 @@ __device__ __forceinline__ void stage_tile(const CaseDev& C, const StageArgs& A,
       R[s] = P[s * NC + c0 + st] - Hs[s * G.nhs + hr];
     }
     const double* fm = d == 0 ? C.fm1 : (d == 1 ? C.fm2 : C.fm3);
-    int64_t NFg = d == 0 ? C.NF1 : (d == 1 ? C.NF2 : C.NF3);
     int64_t fg = d == 0 ? B.f1off + i + (int64_t)(B.n1 + 1) * ((j - 1) + (int64_t)B.n2 * (k - 1))
                : d == 1 ? B.f2off + (i - 1) + (int64_t)B.n1 * (j + (int64_t)(B.n2 + 1) * (k - 1))
                         : B.f3off + (i - 1) + (int64_t)B.n1 * ((j - 1) + (int64_t)B.n2 * k);
-    conv_face_lr<NS, NR, RS>(T, C.rs, C.mco, L, R, fm[fg], fm[NFg + fg], fm[2 * NFg + fg], fm[3 * NFg + fg], res);
+    conv_face_lr<NS, NR, RS>(T, C.rs, C.mco, L, R, fm[4 * fg], fm[4 * fg + 1], fm[4 * fg + 2], fm[4 * fg + 3], res);
 #pragma unroll
     for (int s = 0; s < NP; ++s) Fb[s * NF + f] = res[s];
   }

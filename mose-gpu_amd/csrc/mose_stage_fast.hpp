@@ -110,7 +110,7 @@ __device__ __forceinline__ void visc_face_lds(const CaseDev& C, const double* Pl
 #pragma unroll
     for (int y = 0; y < 3; ++y) {
       if constexpr (MG) Mav[x][y] = mg[x + 3 * y];
-      else Mav[x][y] = 0.5 * (C.m[(int64_t)(x + 3 * y) * NC + c0] + C.m[(int64_t)(x + 3 * y) * NC + c1]);
+      else Mav[x][y] = 0.5 * (C.m[9 * c0 + x + 3 * y] + C.m[9 * c1 + x + 3 * y]);
     }
   const double drho = ft.rho, dmil = ft.mil, ird = rcp_nr(drho);
   double mie = 0.0;
@@ -285,11 +285,6 @@ __device__ __forceinline__ void stage_tile_fast(const CaseDev& C, const StageArg
   constexpr bool MST = VISC && NS == 1 && NR == 0 && STI == 8 && STJ == 8 && STK == 4;
   double* Fb = Cc + FC::n * NB + (MST ? 128 : 0);   // [NP][nslot]
   const int64_t si = 1, sj = B.pi, sk = (int64_t)B.pi * B.pj;
-  // The i-stride of the viscous faces' cell-metric loads, for one species without RANS as a run-time value (B.pi is
-  // never 0): with the constant 1 the compiler merges each pair m[c0], m[c0 + 1] into one 16-byte load and issues the
-  // nine merged loads one after another, each waiting for the last (3.4 % of the 256^3 Taylor-Green stage); as two
-  // 8-byte loads they are issued together, as on the j- and k-faces.
-  const int64_t siv = (NS == 1 && NR == 0) ? (int64_t)(B.pi > 0) : si;
 
   // ---------------- phase L: the primitives of the box and the slabs into LDS ----------------
   // up to LU cells per thread per pass, every load of the pass issued before the first LDS store (LU x NP doubles
@@ -423,11 +418,10 @@ __device__ __forceinline__ void stage_tile_fast(const CaseDev& C, const StageArg
     const double* dlp = C.dl + (int64_t)d * NC;
     const double dLL = dlp[c0 - st], dL = dlp[c0], dR = dlp[c0 + st], dRR = dlp[c0 + 2 * st];
     const double* fm = d == 0 ? C.fm1 : (d == 1 ? C.fm2 : C.fm3);
-    const int64_t NFg = d == 0 ? C.NF1 : (d == 1 ? C.NF2 : C.NF3);
     const int64_t fg = d == 0 ? B.f1off + i + (int64_t)(B.n1 + 1) * ((j - 1) + (int64_t)B.n2 * (k - 1))
                      : d == 1 ? B.f2off + (i - 1) + (int64_t)B.n1 * (j + (int64_t)(B.n2 + 1) * (k - 1))
                               : B.f3off + (i - 1) + (int64_t)B.n1 * ((j - 1) + (int64_t)B.n2 * k);
-    const double fnx = fm[fg], fny = fm[NFg + fg], fnz = fm[2 * NFg + fg], fa = fm[3 * NFg + fg];
+    const double fnx = fm[4 * fg], fny = fm[4 * fg + 1], fnz = fm[4 * fg + 2], fa = fm[4 * fg + 3];
     const double i0 = rcp_nr(0.5 * (dLL + dL)), i1 = rcp_nr(0.5 * (dL + dR)), i2 = rcp_nr(0.5 * (dR + dRR));
     const double hL = 0.5 * dL, hR = 0.5 * dR;
     double L[NP], R[NP], res[NP];
@@ -485,10 +479,10 @@ __device__ __forceinline__ void stage_tile_fast(const CaseDev& C, const StageArg
     const int64_t cm = inb ? row(B, mi, mj, mk) : 0;
     if (tid < 256) {
 #pragma unroll
-      for (int q = 0; q < 5; ++q) Pl[q * NX + NB + l] = inb ? C.m[(int64_t)q * NC + cm] : 0.0;
+      for (int q = 0; q < 5; ++q) Pl[q * NX + NB + l] = inb ? C.m[9 * cm + q] : 0.0;
     } else {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) mreg[q] = inb ? C.m[(int64_t)(5 + q) * NC + cm] : 0.0;
+      for (int q = 0; q < 4; ++q) mreg[q] = inb ? C.m[9 * cm + 5 + q] : 0.0;
     }
   }
 
@@ -522,11 +516,10 @@ __device__ __forceinline__ void stage_tile_fast(const CaseDev& C, const StageArg
       const int k1 = (a + 1 - (d == 0)) + CI * ((b + 1 - (d == 1)) + CJ * (c + 1 - (d == 2)));
       const int64_t c0 = row(B, i, j, k);
       const double* fm = d == 0 ? C.fm1 : (d == 1 ? C.fm2 : C.fm3);
-      const int64_t NFg = d == 0 ? C.NF1 : (d == 1 ? C.NF2 : C.NF3);
       const int64_t fg = d == 0 ? B.f1off + i + (int64_t)(B.n1 + 1) * ((j - 1) + (int64_t)B.n2 * (k - 1))
                        : d == 1 ? B.f2off + (i - 1) + (int64_t)B.n1 * (j + (int64_t)(B.n2 + 1) * (k - 1))
                                 : B.f3off + (i - 1) + (int64_t)B.n1 * ((j - 1) + (int64_t)B.n2 * k);
-      const double fnx = fm[fg], fny = fm[NFg + fg], fnz = fm[2 * NFg + fg], fa = fm[3 * NFg + fg];
+      const double fnx = fm[4 * fg], fny = fm[4 * fg + 1], fnz = fm[4 * fg + 2], fa = fm[4 * fg + 3];
       // the tile cells of the face (lower lo, upper up) and the face-averaged metric
       const int lo = (a - (d == 0)) + 8 * ((b - (d == 1)) + 8 * (c - (d == 2)));
       const int up = lo + (d == 0 ? 1 : (d == 1 ? 8 : 64));
@@ -539,7 +532,7 @@ __device__ __forceinline__ void stage_tile_fast(const CaseDev& C, const StageArg
         const int lin = side ? lo : up;
         const int64_t cout = side ? c0 + (d == 0 ? si : (d == 1 ? sj : sk)) : c0;
 #pragma unroll
-        for (int q = 0; q < 9; ++q) mg[q] = 0.5 * (mt(q, lin) + C.m[(int64_t)q * NC + cout]);
+        for (int q = 0; q < 9; ++q) mg[q] = 0.5 * (mt(q, lin) + C.m[9 * cout + q]);
       }
       double res[NP];
       if (d == 0) visc_face_lds<NS, NR, 0, true>(C, Pl, NX, Cc, NB, k1, k1 + 1, CI, CI * CJ, c0, c0, fnx, fny, fnz, fa, res, mg);
@@ -577,13 +570,12 @@ __device__ __forceinline__ void stage_tile_fast(const CaseDev& C, const StageArg
       const int k1 = (a + 1 - (d == 0)) + CI * ((b + 1 - (d == 1)) + CJ * (c + 1 - (d == 2)));
       const int64_t c0 = row(B, i, j, k);
       const double* fm = d == 0 ? C.fm1 : (d == 1 ? C.fm2 : C.fm3);
-      const int64_t NFg = d == 0 ? C.NF1 : (d == 1 ? C.NF2 : C.NF3);
       const int64_t fg = d == 0 ? B.f1off + i + (int64_t)(B.n1 + 1) * ((j - 1) + (int64_t)B.n2 * (k - 1))
                        : d == 1 ? B.f2off + (i - 1) + (int64_t)B.n1 * (j + (int64_t)(B.n2 + 1) * (k - 1))
                                 : B.f3off + (i - 1) + (int64_t)B.n1 * ((j - 1) + (int64_t)B.n2 * k);
-      const double fnx = fm[fg], fny = fm[NFg + fg], fnz = fm[2 * NFg + fg], fa = fm[3 * NFg + fg];
+      const double fnx = fm[4 * fg], fny = fm[4 * fg + 1], fnz = fm[4 * fg + 2], fa = fm[4 * fg + 3];
       double res[NP];
-      if (d == 0) visc_face_lds<NS, NR, 0>(C, Pl, NX, Cc, NB, k1, k1 + 1, CI, CI * CJ, c0, c0 + siv, fnx, fny, fnz, fa, res);
+      if (d == 0) visc_face_lds<NS, NR, 0>(C, Pl, NX, Cc, NB, k1, k1 + 1, CI, CI * CJ, c0, c0 + si, fnx, fny, fnz, fa, res);
       else if (d == 1) visc_face_lds<NS, NR, 1>(C, Pl, NX, Cc, NB, k1, k1 + CI, 1, CI * CJ, c0, c0 + sj, fnx, fny, fnz, fa, res);
       else visc_face_lds<NS, NR, 2>(C, Pl, NX, Cc, NB, k1, k1 + CI * CJ, 1, CI, c0, c0 + sk, fnx, fny, fnz, fa, res);
 #pragma unroll
