@@ -255,6 +255,19 @@ __device__ __forceinline__ void stage_tile(const CaseDev& C, const StageArgs& A,
 #pragma unroll
     for (int s = 0; s < NP; ++s) Fb[s * NF + f] = res[s];
   }
+  // the thread's cell; its step base and volume are loaded ahead of the last barrier before phase D
+  int ca = tid % TI, cb = (tid / TI) % TJ, cc = tid / (TI * TJ);
+  int ci = tl.i0 + ca, cj = tl.j0 + cb, ck = tl.k0 + cc;
+  bool mine = (tid < TI * TJ * TK) && ci <= B.n1 && cj <= B.n2 && ck <= B.n3;
+  double po[NP], vol = 1.0;
+  auto base = [&]() {
+    if (!mine) return;
+    const int64_t c0 = row(B, ci, cj, ck);
+#pragma unroll
+    for (int s = 0; s < NP; ++s) po[s] = C.PO[s * NC + c0];
+    vol = C.vol[c0];
+  };
+  if (!VISC) base();
   __syncthreads();
   if (VISC) {
     // the half-slopes are dead: region 0 now holds (rho, 1/rho, T) of the tile and its one-cell halo
@@ -277,9 +290,6 @@ __device__ __forceinline__ void stage_tile(const CaseDev& C, const StageArgs& A,
   }
 
   // ---------------- phase B: convective sums ----------------
-  int ca = tid % TI, cb = (tid / TI) % TJ, cc = tid / (TI * TJ);
-  int ci = tl.i0 + ca, cj = tl.j0 + cb, ck = tl.k0 + cc;
-  bool mine = (tid < TI * TJ * TK) && ci <= B.n1 && cj <= B.n2 && ck <= B.n3;
   int sIm = ca + (TI + 1) * (cb + TJ * cc), sJm = NI + ca + TI * (cb + (TJ + 1) * cc), sKm = NI + NJ + ca + TI * (cb + TJ * cc);
   int sIp = sIm + 1, sJp = sJm + TI, sKp = sKm + TI * TJ;
   double tmp[NP];
@@ -320,6 +330,7 @@ __device__ __forceinline__ void stage_tile(const CaseDev& C, const StageArgs& A,
 #pragma unroll
       for (int s = 0; s < NP; ++s) Fb[s * NF + f] = res[s];
     }
+    base();
     __syncthreads();
     if (mine) {
 #pragma unroll
@@ -353,10 +364,13 @@ __device__ __forceinline__ void stage_tile(const CaseDev& C, const StageArgs& A,
         tmp[s] = tmp[s] + C.binc[(int64_t)(NP + s) * C.NBP + pos];
       }
     }
-    int64_t c0 = row(B, ci, cj, ck);
-    double p[NP], po[NP], out[NP];
+    const int64_t c0 = row(B, ci, cj, ck);
+    double p[NP], out[NP];
 #pragma unroll
-    for (int s = 0; s < NP; ++s) { p[s] = P[s * NC + c0]; po[s] = C.PO[s * NC + c0]; }
+    for (int s = 0; s < NP; ++s) {
+      if (VISC) p[s] = cache[(3 + s) * G.ncache + (ca + 1) + (TI + 2) * ((cb + 1) + (TJ + 2) * (cc + 1))];
+      else p[s] = P[s * NC + c0];
+    }
     double Tseed;
     if (VISC) {
       const int CI = TI + 2, CJ = TJ + 2;
@@ -374,8 +388,8 @@ __device__ __forceinline__ void stage_tile(const CaseDev& C, const StageArgs& A,
       double rho = cache[(ca + 1) + (TI + 2) * ((cb + 1) + (TJ + 2) * (cc + 1))];
       cell_sa<NS, NR>(C, B, ci, cj, ck, c0, rho, cell_mil<NS>(T, p, rho, Tseed), tmp);
     }
-    if (C.prim) update_cell_prim<NS, NR>(T, p, po, tmp, C.vol[c0], *C.dt, C.strang, A.rkc, out);
-    else update_cell<NS, NR>(T, p, po, tmp, C.vol[c0], *C.dt, C.strang, A.rkc, Tseed, out);
+    if (C.prim) update_cell_prim<NS, NR>(T, p, po, tmp, vol, *C.dt, C.strang, A.rkc, out);
+    else update_cell<NS, NR>(T, p, po, tmp, vol, *C.dt, C.strang, A.rkc, Tseed, out);
     bool good = out[V::np] >= 0.0;
 #pragma unroll
     for (int s = 0; s < NP; ++s) good = good && isfinite(out[s]);

@@ -438,12 +438,35 @@ __device__ __forceinline__ void stage_tile_fast(const CaseDev& C, const StageArg
 #pragma unroll
     for (int s = 0; s < NP; ++s) Fb[s * NF + f] = res[s];
   }
-  __syncthreads();
 
-  // ---------------- phase B: convective sums ----------------
+  // ---------------- loads of the cells, in flight over the barriers ----------------
+  // MST: the tile's metrics, over the barrier after phase A; the step base and volume of the thread's cell (`base`), over
+  // the last barrier before phase D.  256^3 Taylor-Green: 3.49 -> 3.34 ms a stage.  (The first face's geometry over the
+  // barrier before phase A, likewise, made it 3.44.)
   const int ca = tid % TI, cb = (tid / TI) % TJ, cc = tid / (TI * TJ);
   const int ci = tl.i0 + ca, cj = tl.j0 + cb, ck = tl.k0 + cc;
   const bool mine = (tid < TI * TJ * TK) && ci <= B.n1 && cj <= B.n2 && ck <= B.n3;
+  const int64_t c0 = mine ? row(B, ci, cj, ck) : 0;
+  double po[NP], vol = 1.0;
+  auto base = [&]() {
+    if (!mine) return;
+#pragma unroll
+    for (int s = 0; s < NP; ++s) po[s] = C.PO[s * NC + c0];
+    vol = C.vol[c0];
+  };
+  if constexpr (!VISC) base();
+  double mreg[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  if constexpr (MST) {
+    const int l = tid & 255, mi = tl.i0 + (l & 7), mj = tl.j0 + ((l >> 3) & 7), mk = tl.k0 + (l >> 6);
+    if (mi <= B.n1 && mj <= B.n2 && mk <= B.n3) {
+      const double* mp = C.m + 9 * row(B, mi, mj, mk) + (tid < 256 ? 0 : 4);
+#pragma unroll
+      for (int q = 0; q < 5; ++q) mreg[q] = mp[q];
+    }
+  }
+  __syncthreads();
+
+  // ---------------- phase B: convective sums ----------------
   const int sIm = ca + (TI + 1) * (cb + TJ * cc), sJm = NI + ca + TI * (cb + (TJ + 1) * cc),
             sKm = NI + NJ + ca + TI * (cb + TJ * cc);
   const int sIp = sIm + 1, sJp = sJm + TI, sKp = sKm + TI * TJ;
@@ -472,17 +495,10 @@ __device__ __forceinline__ void stage_tile_fast(const CaseDev& C, const StageArg
   // cells in the tile (640 of 896) then take their metric from LDS instead of 18 global loads; the 256 on the tile's
   // sides load the outer cell's.  Threads 0..255 store components 0..4 while phase B runs; threads 256..511 hold
   // 5..8 in registers until phase B's reads of Fb are over.
-  double mreg[4] = {0.0, 0.0, 0.0, 0.0};
   if constexpr (MST) {
-    const int l = tid & 255, mi = tl.i0 + (l & 7), mj = tl.j0 + ((l >> 3) & 7), mk = tl.k0 + (l >> 6);
-    const bool inb = mi <= B.n1 && mj <= B.n2 && mk <= B.n3;
-    const int64_t cm = inb ? row(B, mi, mj, mk) : 0;
     if (tid < 256) {
 #pragma unroll
-      for (int q = 0; q < 5; ++q) Pl[q * NX + NB + l] = inb ? C.m[9 * cm + q] : 0.0;
-    } else {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) mreg[q] = inb ? C.m[9 * cm + 5 + q] : 0.0;
+      for (int q = 0; q < 5; ++q) Pl[q * NX + NB + tid] = mreg[q];
     }
   }
 
@@ -492,7 +508,7 @@ __device__ __forceinline__ void stage_tile_fast(const CaseDev& C, const StageArg
     __syncthreads();
     if (tid >= 256) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) Mx[q * 256 + (tid & 255)] = mreg[q];
+      for (int q = 0; q < 4; ++q) Mx[q * 256 + (tid & 255)] = mreg[1 + q];
     }
     __syncthreads();
     for (int g = tid; g < NF; g += BS) {
@@ -542,6 +558,7 @@ __device__ __forceinline__ void stage_tile_fast(const CaseDev& C, const StageArg
 #pragma unroll
       for (int s = 1; s < NP; ++s) Fb[s * NF + f] = res[s];
     }
+    base();
     __syncthreads();
     if (mine) {
 #pragma unroll
@@ -581,6 +598,7 @@ __device__ __forceinline__ void stage_tile_fast(const CaseDev& C, const StageArg
 #pragma unroll
       for (int s = 0; s < NP; ++s) Fb[s * NF + f] = res[s];
     }
+    base();
     __syncthreads();
     if (mine) {
 #pragma unroll
@@ -614,11 +632,10 @@ __device__ __forceinline__ void stage_tile_fast(const CaseDev& C, const StageArg
         tmp[s] = tmp[s] + C.binc[(int64_t)(NP + s) * C.NBP + pos];
       }
     }
-    const int64_t c0 = row(B, ci, cj, ck);
-    double p[NP], po[NP], out[NP];
+    double p[NP], out[NP];
 #pragma unroll
-    for (int s = 0; s < NP; ++s) { p[s] = Pl[s * NX + kc0]; po[s] = C.PO[s * NC + c0]; }
-    const double w = *C.dt * C.strang * rcp_nr(C.vol[c0]);
+    for (int s = 0; s < NP; ++s) p[s] = Pl[s * NX + kc0];
+    const double w = *C.dt * C.strang * rcp_nr(vol);
     double Tseed;
     if constexpr (VISC) {
       Tseed = Cc[FC::iT * NB + kc0];
@@ -637,7 +654,7 @@ __device__ __forceinline__ void stage_tile_fast(const CaseDev& C, const StageArg
     }
     // the primitive update below nine species (the nine-species kernels take the conservative one only)
     if constexpr (NS < 9) {
-      if (C.prim) update_cell_prim<NS, NR>(T, p, po, tmp, C.vol[c0], *C.dt, C.strang, A.rkc, out);
+      if (C.prim) update_cell_prim<NS, NR>(T, p, po, tmp, vol, *C.dt, C.strang, A.rkc, out);
       else update_cell_nr<NS, NR>(T, p, po, tmp, w, A.rkc, Tseed, out);
     } else {
       update_cell_nr<NS, NR>(T, p, po, tmp, w, A.rkc, Tseed, out);
