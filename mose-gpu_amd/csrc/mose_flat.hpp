@@ -12,7 +12,7 @@
 // 51 KB, and the faces take one pass.  A small case is bound by the length of one thread's chain of loads and operations
 // (load, face, update), a large one by the FP64 units.
 // Stage times, general kernel -> this one (boundary kernel included): shock tube of 1000 cells 22 -> 16 us, Riemann problems of
-// 64^2 20 -> 16 us, 1023^2 285 -> 135 us (FP64 units 43 % busy with a thread per face there, 60 % with one per cell).
+// 64^2 20 -> 16 us, 1023^2 285 -> 135 us (65 us of it FP64 issue; 180 us with a thread per face there).
 #pragma once
 
 #include "mose_stage_fast.hpp"
