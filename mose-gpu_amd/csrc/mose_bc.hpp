@@ -4,7 +4,9 @@
 // The increments of viscous connection and symmetry records read ghost cells of other faces (the transverse neighbours
 // of a cell on a block edge), which made the two kernels a chain.  Here such a neighbour is read from the interior cell
 // that its own record copies (BcNbr holds the rows), or, behind mirror and cubic ghosts, formed again with that record's
-// statements (ghost1), so the records need no order.
+// statements (ghost1).  No record then reads a ghost that another stores, and they need no order: along its normal a
+// planned record that reads its cell's neighbour (connections, symmetry, walls, far field) has a block of two cells or
+// more, so that the neighbour is an interior cell (plan_boundary).
 // A record's own layers stay in registers between the ghost store and the flux.
 //
 // The Euler increment (with the ghosts) and the viscous one of a record are two threads of different workgroups: the
@@ -63,8 +65,7 @@ static __global__ void __launch_bounds__(64) k_bc_geometry(CaseDev C, const BcPl
   geo[BCG_DL * N + t] = dlp[c - 2 * in];
   geo[(BCG_DL + 1) * N + t] = dlp[c - in];
   geo[(BCG_DL + 2) * N + t] = dlp[c];
-  const mose_blk B = C.blk[p.b];
-  geo[(BCG_DL + 3) * N + t] = dlp[(d == 0 ? B.n1 : (d == 1 ? B.n2 : B.n3)) > 1 ? c + in : c];
+  geo[(BCG_DL + 3) * N + t] = dlp[c + in];
   if (!C.visc) return;
   for (int q = 0; q < 9; ++q) geo[(BCG_M + q) * N + t] = 0.5 * (C.m[9 * c + q] + C.m[9 * (c - in) + q]);
 }

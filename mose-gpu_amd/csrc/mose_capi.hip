@@ -422,9 +422,10 @@ static size_t case_bytes(const Case& c) {
   return b;
 }
 
-// Inviscid cases read no ghost behind the no-flux faces of a direction of one cell: such records are not planned, and
-// their ghosts are filled (with the others, by k_ghost) when the state is downloaded.  On a 1023^2 Riemann problem they
-// are 2.09 of the 2.10 million records, and took a third of a step.
+// Inviscid cases read no ghost behind the no-flux faces of a direction of one cell (where a record on the opposite face
+// would read it, plan_boundary makes no plan): such records are not planned, and their ghosts are filled (with the
+// others, by k_ghost) when the state is downloaded.  On a 1023^2 Riemann problem they are 2.09 of the 2.10 million
+// records, and took a third of a step.
 static bool bc_dead(const Case& c, const mose_bc_record& r) {
   const mose_blk& B = c.blk[r.b];
   const int d = (r.f + 1) / 2;
@@ -445,7 +446,11 @@ static CaseDev make_dev(mose_ctx* ctx, Case& c, const double* Pin, double* Pout)
 static inline unsigned nblocks(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
 
 // The boundary plan (mose_bc.hpp).  Cases of nine species and connections whose transverse maps are not one step along
-// one axis keep k_ghost and k_bcrec (ghost1 forms the first ghost layer next to a cell, no corner).
+// one axis keep k_ghost and k_bcrec (ghost1 forms the first ghost layer next to a cell, no corner).  So do cases with a
+// symmetry record or the receiver of a connection in a direction of one cell: their increments take the neighbour along
+// the normal, which there is the ghost behind the opposite face, and only the order of the two kernels gives them that
+// face's ghost of this stage.  (Walls and far-field faces need more cells along their normal, plan_case; extrapolation
+// and no-flux increments do not read the neighbour.)
 static int plan_boundary(mose_ctx* ctx, Case& c, hipStream_t s) {
   if (c.sc.nsc > 4 || c.rec.empty() || c.NC > 0x7fffffff || std::max({c.NF1, c.NF2, c.NF3, c.NBP}) > 0x7fffffff) return MOSE_OK;
   auto row_of = [&](int b, const int* x) {
@@ -466,6 +471,8 @@ static int plan_boundary(mose_ctx* ctx, Case& c, hipStream_t s) {
     return (r.typ == MOSE_BC_EXTRAPOLATION && extent(r) >= 3) || r.typ == MOSE_BC_WALL_ADIABATIC ||
            r.typ == MOSE_BC_WALL_ISOTHERMAL;
   };
+  for (const auto& r : c.rec)
+    if (extent(r) == 1 && (r.typ == MOSE_BC_SYMMETRY || r.typ == MOSE_BC_CONNECTION)) return MOSE_OK;
   // the order: by type, direction and side (the low bits of meta), the records of each in their own order
   auto key = [&](const mose_bc_record& r) {
     return (unsigned)r.typ | (unsigned)((r.f + 1) / 2 - 1) << BCP_DIR | (unsigned)(r.f % 2) << BCP_ODD;
