@@ -177,7 +177,13 @@ int mose_case_destroy(mose_ctx* ctx, int case_id);
 /* bytes of device memory a case of these blocks takes (the serving loop admits by this figure) */
 int mose_case_bytes(const mose_scheme* scheme, int nb, const int* dims, int nrec, int64_t* bytes);
 
-/* State in and out (pack_P_to_flat / unpack_flat_to_P, MOSE_Field_m.f90:171-194,334-369). */
+/* State in and out (pack_P_to_flat / unpack_flat_to_P, MOSE_Field_m.f90:171-194,334-369).
+ * Ghost rows of a download.  Before the first step: as uploaded.  After steps the interior is the new state, while the
+ * ghosts behind the faces are those that the last step's first stage filled, the closures of the state that this step
+ * started from (with Strang-split chemistry, that its second half started from).  One exception: the fused paths (MOSE_PATH_FUSED, MOSE_PATH_FAST) leave out the ghosts behind no-flux
+ * faces (type 0) of a direction of one cell in inviscid cases, where no stage reads them; a download of such a case fills
+ * the ghosts of all its faces, from the state that it returns.  Every step fills the ghosts that it reads, so uploaded
+ * ghost rows do not enter a result. */
 int mose_state_upload(mose_ctx* ctx, int case_id, const double* P);
 int mose_state_download(mose_ctx* ctx, int case_id, double* P);
 

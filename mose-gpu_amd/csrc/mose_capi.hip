@@ -912,6 +912,8 @@ static void launch_ghosts(Case& c, const CaseDev& D, hipStream_t s) {
   k_ghost<NS, NR><<<nblocks((int64_t)c.rec.size(), 256), 256, 0, s>>>(D);
 }
 
+// before a download: where the steps left out the ghosts of dead records, those of all records, from the state returned
+// (the state that the last step started from is gone)
 static int fill_dead_ghosts(mose_ctx* ctx, Case& c) {
   if (!c.dead_stale || c.ndead == 0) return MOSE_OK;
   CaseDev D = make_dev(ctx, c, c.P0, c.PA);
@@ -1158,10 +1160,8 @@ static int run_steps(mose_ctx* ctx, Case& c, int nsteps) {
     }
     c.dt_valid = fused;
   }
-  if (fused && nsteps > 0) {
-    k_dt_final<<<1, 64, 0, s>>>(c.dtnext, c.dt, nullptr, 0);   // between calls dt is the next step's
-    c.dead_stale = true;
-  }
+  if (fused && nsteps > 0) k_dt_final<<<1, 64, 0, s>>>(c.dtnext, c.dt, nullptr, 0);   // between calls dt is the next step's
+  if (nsteps > 0) c.dead_stale = fused;   // the plain path fills every ghost
   HIPCHK(ctx, hipGetLastError());
   if (c.timing && iev > 0) {
     HIPCHK(ctx, hipStreamSynchronize(s));
