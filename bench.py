@@ -33,12 +33,14 @@ def algorithmic_bytes_per_cell_stage(nprim: int, viscous: bool, rans: bool) -> i
     return 8 * (3 * nprim + G)
 
 
-def profiled_counts(n: int, nprim: int, viscous: bool, tile, path: str = "fused") -> tuple[int | None, int | None]:
-    """(HBM bytes, VALU wavefront instructions) per stage launch, measured by rocprofv3 counters for this workload
-    (profiles/*_traffic.txt), or None where the workload has not been profiled."""
+def profiled_counts(n: int, nprim: int, viscous: bool, tile, path: str = "fused",
+                    records: str = "traffic") -> tuple[int | None, int | None]:
+    """(HBM bytes, VALU wavefront instructions) per stage launch, measured by rocprofv3 counters for this workload, or
+    None where the workload has not been profiled.  records: "counters", the present kernels (profiles/*_counters.txt),
+    or "traffic", the builds that those records name (profiles/*_traffic.txt)."""
     kern = "k_stage" if path == "fused" else f"k_stage_{path}"
     key = (kern, str(n), str(nprim), str(int(viscous)), "x".join(str(t) for t in tile))
-    for f in sorted((REPO / "profiles").glob("*_traffic.txt")):
+    for f in sorted((REPO / "profiles").glob(f"*_{records}.txt")):
         for line in f.read_text().splitlines():
             w = line.split()
             if len(w) >= 6 and not line.startswith("#") and tuple(w[:5]) == key:
@@ -113,7 +115,7 @@ def chemistry_leg(ncell: int, cpu_cells: int, threads: int, radau_cells: int = 0
            "steps_max": int(nstep.max()), "rhs_evals": int(rep.rhs_total), "failed": int((idid < 0).sum()),
            "workload": "H2-O2-N2 9 species, 17 Arrhenius + 2 Troe, 1 atm, T U[900,2500] K, phi U[0.5,2], "
                        "dt 1e-6 s, RODAS rtol 1e-8 atol 1e-12"}
-    per = chem_valu_per_attempt()
+    per = chem_valu_per_attempt("counters")
     if per:
         # FP64 VALU issue: a wave64 instruction takes 4 cycles of one SIMD (1,024 SIMDs at 2.4 GHz); the share of the
         # launch that the profiled instructions per step attempt, times this launch's attempts, take to issue
@@ -216,10 +218,10 @@ def shock_tube_leg(threads: int):
     return res
 
 
-def chem_valu_per_attempt() -> float | None:
-    """VALU wavefront instructions per RODAS step attempt of k_chem, from the profiled counters
-    (profiles/*_traffic.txt key k_chem_valu_per_attempt), or None."""
-    for f in sorted((REPO / "profiles").glob("*_traffic.txt")):
+def chem_valu_per_attempt(records: str = "traffic") -> float | None:
+    """VALU wavefront instructions per RODAS step attempt, from the profiled counters (key k_chem_valu_per_attempt), or
+    None; records as in profiled_counts."""
+    for f in sorted((REPO / "profiles").glob(f"*_{records}.txt")):
         for line in f.read_text().splitlines():
             w = line.split()
             if len(w) >= 2 and w[0] == "k_chem_valu_per_attempt":
@@ -400,7 +402,8 @@ def main():
     value = cells * args.steps / elapsed
     B = algorithmic_bytes_per_cell_stage(case.nprim, True, False)
     achieved = (B * cells) / (ms_avg * 1e-3) / 1e9 if ms_avg > 0 else None
-    traffic, valu = profiled_counts(args.n, case.nprim, True, chosen, args.path) if fused_like else (None, None)
+    traffic, valu = (profiled_counts(args.n, case.nprim, True, chosen, args.path, "counters") if fused_like
+                     else (None, None))
     roofline = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": (achieved / HBM_PEAK_GBS) if achieved else None,
                 "traffic": traffic,

@@ -42,3 +42,14 @@ def test_algorithmic_bytes():
 
 def test_chemistry_instruction_count_from_the_profile():
     assert bench.chem_valu_per_attempt() == 3921.0
+
+
+def test_counts_of_the_present_kernels():
+    """bench.py's figures of the kernels in the tree come from records of their own: a shape that they were not profiled
+    at has none, whatever an earlier build's record holds."""
+    traffic, valu = bench.profiled_counts(256, 5, True, (8, 8, 4), "fast", "counters")
+    assert traffic == 8566672018 and valu == 1132166583
+    traffic, valu = bench.profiled_counts(256, 5, True, (8, 8, 4), "fused", "counters")
+    assert traffic == 8563619224 and valu == 1938494805
+    assert bench.profiled_counts(256, 5, True, (8, 8, 8), "fused", "counters") == (None, None)
+    assert bench.chem_valu_per_attempt("counters") == 1994.0
