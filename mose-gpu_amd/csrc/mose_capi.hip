@@ -1019,6 +1019,9 @@ static int set_tiles(mose_ctx* ctx, Case& c, int TI, int TJ, int TK) {
     return fail(ctx, MOSE_ERR_ARG, "tile " + std::to_string(TI) + "x" + std::to_string(TJ) + "x" + std::to_string(TK) +
                                        " needs " + std::to_string(stage_lds(c, TI, TJ, TK)) + " B of LDS, the device allows " +
                                        std::to_string(ctx->max_lds));
+  // (170 KB of LDS for the smallest one, 8 x 8 x 4, whatever the device allows: their parity kernels are not built)
+  if (c.sc.nsc >= 9 && c.sc.viscous && TI * TJ * TK > 128)
+    return fail(ctx, MOSE_ERR_ARG, "a viscous tile of nine species holds 128 cells");
   // tiles block by block, in super-tiles of 4 x 4 x 4 tiles (i fastest inside a super-tile and between them):
   // neighbouring tiles run close together in time and share the L2 of their XCD (1.4 % faster than plain i-fastest
   // order on the 256^3 Taylor-Green case)

@@ -442,11 +442,13 @@ template <int NS, int NR, int BS, int SH>
 void launch_stage_shape(const CaseDev& D, const StageArgs& A, int rs, bool visc, unsigned grid, size_t lds,
                         hipStream_t s) {
   if (visc) {
-    if (rs == MOSE_RS_LMROE) k_stage<NS, NR, true, MOSE_RS_LMROE, BS, SH><<<grid, BS, lds, s>>>(D, A);
-    else if (rs == MOSE_RS_AUSMP) k_stage<NS, NR, true, MOSE_RS_AUSMP, BS, SH><<<grid, BS, lds, s>>>(D, A);
-    else if (rs == MOSE_RS_HLLE) k_stage<NS, NR, true, MOSE_RS_HLLE, BS, SH><<<grid, BS, lds, s>>>(D, A);
-    else if (rs == MOSE_RS_SLAU) k_stage<NS, NR, true, MOSE_RS_SLAU, BS, SH><<<grid, BS, lds, s>>>(D, A);
-    else k_stage<NS, NR, true, MOSE_RS_HLLC, BS, SH><<<grid, BS, lds, s>>>(D, A);
+    if constexpr (NS < 9 || BS == 256) {     // nine species: no larger viscous tile passes set_tiles
+      if (rs == MOSE_RS_LMROE) k_stage<NS, NR, true, MOSE_RS_LMROE, BS, SH><<<grid, BS, lds, s>>>(D, A);
+      else if (rs == MOSE_RS_AUSMP) k_stage<NS, NR, true, MOSE_RS_AUSMP, BS, SH><<<grid, BS, lds, s>>>(D, A);
+      else if (rs == MOSE_RS_HLLE) k_stage<NS, NR, true, MOSE_RS_HLLE, BS, SH><<<grid, BS, lds, s>>>(D, A);
+      else if (rs == MOSE_RS_SLAU) k_stage<NS, NR, true, MOSE_RS_SLAU, BS, SH><<<grid, BS, lds, s>>>(D, A);
+      else k_stage<NS, NR, true, MOSE_RS_HLLC, BS, SH><<<grid, BS, lds, s>>>(D, A);
+    }
   } else {
     if (rs == MOSE_RS_LMROE) k_stage<NS, NR, false, MOSE_RS_LMROE, BS, SH><<<grid, BS, lds, s>>>(D, A);
     else if (rs == MOSE_RS_AUSMP) k_stage<NS, NR, false, MOSE_RS_AUSMP, BS, SH><<<grid, BS, lds, s>>>(D, A);
@@ -461,15 +463,16 @@ void launch_stage_tiles(const CaseDev& D, const StageArgs& A, int rs, bool visc,
                         hipStream_t s) {
   const int TI = A.TI, TJ = A.TJ, TK = A.TK;
   if constexpr (NS >= 9) {
-    // nine species: the 8 x 8 x 4 and 8 x 8 x 8 tiles do not fit the LDS, every shape is read at run time
+    // nine species: the 8 x 8 x 4 and 8 x 8 x 8 tiles do not fit the LDS, every shape is read at run time; viscous tiles
+    // hold 128 cells (set_tiles)
     if (TI * TJ * TK == 128) launch_stage_shape<NS, NR, 256, 0>(D, A, rs, visc, grid, lds, s);
     else launch_stage_shape<NS, NR, 512, 0>(D, A, rs, visc, grid, lds, s);
-    return;
+  } else {
+    if (TI * TJ * TK == 128) launch_stage_shape<NS, NR, 256, 0>(D, A, rs, visc, grid, lds, s);
+    else if (TI == 8 && TJ == 8 && TK == 4) launch_stage_shape<NS, NR, 512, 1>(D, A, rs, visc, grid, lds, s);
+    else if (TI == 8 && TJ == 8 && TK == 8) launch_stage_shape<NS, NR, 512, 2>(D, A, rs, visc, grid, lds, s);
+    else launch_stage_shape<NS, NR, 512, 0>(D, A, rs, visc, grid, lds, s);
   }
-  if (TI * TJ * TK == 128) launch_stage_shape<NS, NR, 256, 0>(D, A, rs, visc, grid, lds, s);
-  else if (TI == 8 && TJ == 8 && TK == 4) launch_stage_shape<NS, NR, 512, 1>(D, A, rs, visc, grid, lds, s);
-  else if (TI == 8 && TJ == 8 && TK == 8) launch_stage_shape<NS, NR, 512, 2>(D, A, rs, visc, grid, lds, s);
-  else launch_stage_shape<NS, NR, 512, 0>(D, A, rs, visc, grid, lds, s);
 }
 
 // instantiated per (NS, NR) in mose_stage.hip, one translation unit each
