@@ -233,7 +233,8 @@ int mose_case_state_hash(mose_ctx* ctx, int case_id, uint64_t* h_lo, uint64_t* h
  * further: Noh87's cold gas moves by ~2e-11 under contraction), not bit for bit.
  * A tile holds 128, 256 or 512 cells
  * (ti * tj * tk); ti = tj = tk = 0 autotunes the tile (each candidate timed on the case itself, the state left
- * unchanged).  timing = 1 records HIP events around
+ * unchanged), except for nine species on MOSE_PATH_FAST, where the autotuner returns MOSE_ERR_ARG: it once ended in a
+ * GPU memory fault whose cause is not known.  timing = 1 records HIP events around
  * every stage kernel of the following step calls (mose_case_timing).  No reference counterpart (launch tuning). */
 enum { MOSE_PATH_FUSED = 0, MOSE_PATH_PLAIN = 1, MOSE_PATH_FAST = 2 };
 typedef struct {

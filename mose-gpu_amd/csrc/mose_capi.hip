@@ -1236,6 +1236,10 @@ extern "C" int mose_case_tune(mose_ctx* ctx, int id, const mose_tuning* t, mose_
     return fail(ctx, MOSE_ERR_ARG, "implicit residual smoothing runs on the plain path (MOSE_PATH_PLAIN)");
   if (t->path == MOSE_PATH_FAST && c->sc.nsc == 9 && c->sc.integration == MOSE_INT_PRIM)
     return fail(ctx, MOSE_ERR_ARG, "the performance path's nine-species kernels take the conservative update only");
+  // this autotune once ended in a GPU memory fault whose cause is not known
+  if (t->path == MOSE_PATH_FAST && c->sc.nsc == 9 && t->ti == 0 && t->tj == 0 && t->tk == 0)
+    return fail(ctx, MOSE_ERR_ARG, "the autotuner is off for nine species on the performance path (a GPU fault without a "
+                                   "known cause): give the tile, or take the parity path");
   HIPCHK(ctx, hipSetDevice(ctx->device));
   c->path = t->path;
   c->timing = t->timing != 0;

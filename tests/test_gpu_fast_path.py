@@ -127,9 +127,9 @@ def test_fast_riemann2d(gpu_ready):
 
 @pytest.mark.skip(reason="a GPU memory fault (aperture violation, reported in k_bcrec<9,0>) during this test's autotune "
                          "on a build with a batched phase-L load loop for nine species and a compacted record list; no "
-                         "cause was found by reading the code, both changes were taken out (the nine-species kernels are "
-                         "again instruction for instruction those of the build that passed this test), and the case "
-                         "stays off the GPU until a cause is shown")
+                         "cause was found by reading the code and both changes were taken out; the nine-species kernels "
+                         "have changed since without a run of this test, mose_case_tune refuses the autotune, and the "
+                         "case stays off the GPU until a cause is shown")
 def test_fast_reacting_box(gpu_ready):
     from mosegpu import Context, DeviceCase, DeviceChem
     mech = chem.h2_air_mechanism()
@@ -153,3 +153,21 @@ def test_fast_reacting_box(gpu_ready):
     # and the next step's dt follows the state
     assert abs(rep.time - dts.sum()) <= 1e-8 * dts.sum()
     assert fast_error(case, Pg, Po, f"fast path: reacting box 12x10x8 tile {chosen} x 3 Strang steps") <= 1e-8
+
+
+def test_nine_species_autotune_is_refused(gpu_ready):
+    """Refused on the host, before any launch, with the case's path and tile as they were."""
+    from mosegpu import Context, DeviceCase, MoseError
+    case = cases.reacting_box((6, 5, 4), viscous=True)
+    ctx = Context(case.tables)
+    dc = DeviceCase(ctx, case)
+    dc.upload(case.P)
+    dc.tune(mosegpu.PATH_FUSED, (16, 4, 2))
+    with pytest.raises(MoseError, match="autotuner is off"):
+        dc.tune(FAST, (0, 0, 0))
+    dc.step(1)
+    Pg = dc.download()
+    dc.destroy(); ctx.close()
+    Po = case.P.copy()
+    OracleCase(case).step(Po, 1)
+    assert np.array_equal(case.layout.interior(Pg, 0), case.layout.interior(Po, 0))
