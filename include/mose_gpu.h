@@ -246,6 +246,11 @@ typedef struct {
 } mose_tuning;
 int mose_case_tune(mose_ctx* ctx, int case_id, const mose_tuning* tuning, mose_tuning* chosen);
 
+/* LDS bytes that a workgroup of the stage kernels takes for a tile of ti x tj x tk cells of such a case on a path (0 on
+ * MOSE_PATH_PLAIN): mose_case_tune refuses a tile above the device's limit (lds_per_block of mose_ctx_info).  Needs no
+ * device. */
+int mose_tile_lds(const mose_scheme* scheme, int path, int ti, int tj, int tk, int64_t* bytes);
+
 /* Device time of the stage kernels of the last timed step call: average per launch, total, launch count. */
 int mose_case_timing(mose_ctx* ctx, int case_id, double* ms_stage_avg, double* ms_stage_total, int64_t* launches);
 

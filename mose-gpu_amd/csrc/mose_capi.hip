@@ -1012,6 +1012,17 @@ static size_t stage_lds_(int nprim, bool visc, int TI, int TJ, int TK) {
   return stage_lds(c, TI, TJ, TK);
 }
 
+extern "C" int mose_tile_lds(const mose_scheme* sc, int path, int ti, int tj, int tk, int64_t* bytes) {
+  if (!sc || !bytes || ti < 1 || tj < 1 || tk < 1 || ti > 512 || tj > 512 || tk > 512) return MOSE_ERR_ARG;
+  if (path != MOSE_PATH_FUSED && path != MOSE_PATH_PLAIN && path != MOSE_PATH_FAST) return MOSE_ERR_ARG;
+  Case c;
+  c.sc = *sc;
+  c.nprim = sc->nsc + 4 + sc->nrans;
+  c.path = path;
+  *bytes = path == MOSE_PATH_PLAIN ? 0 : (int64_t)(stage_lds(c, ti, tj, tk) + kStaticLds);
+  return MOSE_OK;
+}
+
 static int set_tiles(mose_ctx* ctx, Case& c, int TI, int TJ, int TK) {
   if (TI < 1 || TJ < 1 || TK < 1 || (TI * TJ * TK != 128 && TI * TJ * TK != 256 && TI * TJ * TK != 512))
     return fail(ctx, MOSE_ERR_ARG, "a tile holds 128, 256 or 512 cells");

@@ -157,6 +157,7 @@ def lib() -> C.CDLL:
     L.mose_case_state_hash.argtypes = [vp, ip, C.POINTER(C.c_uint64), C.POINTER(C.c_uint64)]
     L.mose_case_timing.argtypes = [vp, ip, dp, dp, C.POINTER(C.c_int64)]
     L.mose_case_tune.argtypes = [vp, ip, C.POINTER(Tuning), C.POINTER(Tuning)]
+    L.mose_tile_lds.argtypes = [C.POINTER(Scheme), ip, ip, ip, ip, C.POINTER(C.c_int64)]
     L.mose_bandwidth_probe.argtypes = [vp, C.c_int64, ip, dp]
     L.mose_ctx_info.argtypes = [vp, C.POINTER(C.c_int64), C.POINTER(C.c_int64), C.POINTER(C.c_int), C.POINTER(C.c_int)]
     L.mose_chem_create.argtypes = [vp, C.POINTER(MechanismStruct), C.c_int64, C.POINTER(C.c_int)]
@@ -178,7 +179,7 @@ def lib() -> C.CDLL:
                  "mose_case_tune", "mose_bandwidth_probe", "mose_ctx_info", "mose_chem_create", "mose_chem_destroy",
                  "mose_chem_upload", "mose_chem_download", "mose_chem_advance", "mose_pow_batch",
                  "mose_chem_advance_cells", "mose_case_chem_attach", "mose_case_chem_advance",
-                 "mose_case_chem_report", "mose_wall_distance"):
+                 "mose_case_chem_report", "mose_wall_distance", "mose_tile_lds"):
         getattr(L, name).restype = C.c_int
     _lib_handle = L
     return L

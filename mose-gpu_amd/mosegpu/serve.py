@@ -92,21 +92,39 @@ class ServeStats:
     meta: dict = field(default_factory=dict)
 
 
-def serve_tile(case, path: int):
+def tile_lds(case, path: int, tile) -> int:
+    """LDS bytes of a workgroup of the stage kernels for this tile of the case (mose_tile_lds)."""
+    b = C.c_int64(0)
+    if lib().mose_tile_lds(C.byref(case.scheme), path, *tile, C.byref(b)) != 0:
+        raise ValueError(f"tile {tile}")
+    return int(b.value)
+
+
+def serve_tile(case, path: int, cus: int = 256, lds: int = 160 * 1024):
     """The stage tile of a served case, by rule instead of the autotuner (which would time candidate tiles on every
-    admitted case while the others wait): 8 x 8 x 4 for 3D blocks; 2D ones 16 x 8 x 1, 32 x 8 x 1 from about 100,000 cells
-    on if inviscid (a stage of a 256^2 Riemann case takes 21 against 23 us, of a 1024^2 one 152 against 135 us; a viscous
-    256-cell tile's LDS, most of it for the unused one-cell direction, leaves one workgroup per CU); 1D ones 128 x 1 x 1,
-    256 x 1 x 1 if viscous (1,000 inviscid cells: 16 against 19 us, 200,000 cells: 73 against 72 us)."""
+    admitted case while the others wait): the first of a short list whose workgroup fits the device's LDS (`lds` bytes).
+    3D blocks 8 x 8 x 4 first.  2D ones 16 x 8 x 1 (a larger viscous tile's LDS, most of it for the unused one-cell
+    direction, leaves one workgroup per CU); where the plane kernel runs (inviscid, one species) 32 x 8 x 1 once the
+    smaller tiles are more than its three resident workgroups per compute unit (`cus`): a stage of a 256^2 Riemann case
+    takes 21 against 23 us with the smaller tile, of a 1024^2 one 152 against 135 us.  1D ones 128 x 1 x 1 (1,000 inviscid
+    cells: 16 against 19 us with 256 x 1 x 1, 200,000 cells: 73 against 72 us).  The
+    tiles of 128 cells behind these fit every species count and path."""
     if path == PATH_PLAIN:
         return (0, 0, 0)
     n1, n2, n3 = case.layout.dims[0]
+    sch = case.scheme
+    plane_kernel = not sch.viscous and sch.nsc == 1 and sch.nrans == 0
     if n3 > 1:
-        return (8, 8, 4)
-    large, euler = n1 * n2 > 768 * 128, not case.scheme.viscous
-    if n2 > 1:
-        return (32, 8, 1) if large and euler else (16, 8, 1)
-    return (128, 1, 1) if euler else (256, 1, 1)
+        tiles = [(8, 8, 4), (8, 4, 4)]
+    elif n2 > 1:
+        tiles = [(32, 8, 1)] if plane_kernel and n1 * n2 > 3 * cus * 128 else []
+        tiles += [(16, 8, 1), (8, 4, 4)]
+    else:
+        tiles = [(128, 1, 1), (16, 8, 1), (8, 4, 4)]
+    for t in tiles:
+        if tile_lds(case, path, t) <= lds:
+            return t
+    return tiles[-1]
 
 
 def serve(reqs: list[Request], budget_bytes: int | None = None, quantum: int = 10, path: int = PATH_FUSED,
@@ -123,7 +141,8 @@ def serve(reqs: list[Request], budget_bytes: int | None = None, quantum: int = 1
     def ctx_for(case):
         key = case.name in ("riemann2d",) and "euler" or "ns"
         if key not in ctx_cache:
-            ctx_cache[key] = Context(case.tables)
+            ctx = Context(case.tables)
+            ctx_cache[key] = (ctx, ctx.info())
         return ctx_cache[key]
 
     order = sorted(reqs, key=lambda r: r.arrival)
@@ -178,10 +197,10 @@ def serve(reqs: list[Request], budget_bytes: int | None = None, quantum: int = 1
             if used + nb > budget_bytes and resident:
                 break
             waiting.pop(0)
-            ctx = ctx_for(case)
+            ctx, info = ctx_for(case)
             dc = DeviceCase(ctx, case)
             dc.upload(case.P)
-            dc.tune(path, serve_tile(case, path))
+            dc.tune(path, serve_tile(case, path, info["cus"], info["lds_per_block"]))
             r.admitted = time.perf_counter() - t0
             resident.append({"r": r, "case": case, "dc": dc, "rem": r.steps, "nb": nb, "fly": 0})
             used += nb
@@ -222,7 +241,7 @@ def serve(reqs: list[Request], budget_bytes: int | None = None, quantum: int = 1
             time.sleep(2e-4)
     th.join()
     wall = time.perf_counter() - t0
-    for c in ctx_cache.values():
+    for c, _ in ctx_cache.values():
         c.close()
     lat = np.array([r.done - r.arrival for r in reqs])
     return ServeStats(reqs, wall, len(reqs) / wall, float(np.percentile(lat, 50)), float(np.percentile(lat, 99)),
