@@ -174,7 +174,8 @@ int mose_case_create(mose_ctx* ctx, const mose_scheme* scheme, int nb, const int
                      const double* fm3, int nrec, const mose_bc_record* rec, int nff, const mose_farfield* ff,
                      int* case_id);
 int mose_case_destroy(mose_ctx* ctx, int case_id);
-/* bytes of device memory a case of these blocks takes (the serving loop admits by this figure) */
+/* bytes of device memory that a case of these blocks takes, in the allocator's pages of 2 MiB, every record planned (the
+ * serving loop admits by this figure) */
 int mose_case_bytes(const mose_scheme* scheme, int nb, const int* dims, int nrec, int64_t* bytes);
 
 /* State in and out (pack_P_to_flat / unpack_flat_to_P, MOSE_Field_m.f90:171-194,334-369).

@@ -417,9 +417,16 @@ static size_t case_bytes(const Case& c) {
   b += (std::max<size_t>(c.ff.size(), 1) * sizeof(mose_farfield) + 255) / 256 * 256;
   b += ((size_t)std::max<int64_t>(c.NBP, 1) + 255) / 256 * 256;
   b += 64 * sizeof(double) + 256 + 512;
-  b += c.rec.size() * (sizeof(BcPlan) + sizeof(BcNbr) + (c.sc.viscous ? BCG_VISCOUS : BCG_INVISCID) * d) +
-       (size_t)c.NBP * sizeof(int) + 256;   // the boundary plan (its own allocation)
   return b;
+}
+
+// the boundary plan, an allocation of its own that plan_boundary makes to size: at most this (without the records: dead
+// ones are not planned, some cases make no plan)
+static size_t plan_bytes(const Case& c) {
+  if (c.sc.nsc > 4) return 0;
+  const size_t d = sizeof(double);
+  if (!c.sc.viscous) return c.rec.size() * (sizeof(BcPlan) + BCG_INVISCID * d) + 256;
+  return c.rec.size() * (sizeof(BcPlan) + sizeof(BcNbr) + BCG_VISCOUS * d) + (size_t)c.NBP * sizeof(int) + 256;
 }
 
 // Inviscid cases read no ghost behind the no-flux faces of a direction of one cell (where a record on the opposite face
@@ -572,33 +579,40 @@ static int plan_boundary(mose_ctx* ctx, Case& c, hipStream_t s) {
   return MOSE_OK;
 }
 
+// the allocator hands out 2 MiB pages
+static int64_t page_bytes(size_t b) { return (int64_t)((b + (2u << 20) - 1) / (2u << 20) * (2u << 20)); }
+static constexpr int kHistCap = 4096;
+
+// The case's allocations: the slab, the boundary plan, the norm partials and the tile list (of 8 x 4 x 4
+// tiles, the smallest).
 extern "C" int mose_case_bytes(const mose_scheme* sc, int nb, const int* dims, int nrec, int64_t* bytes) {
   Case c;
-  std::string why;
   if (!bytes) return MOSE_ERR_ARG;
   // sizing does not need the records themselves
   if (!sc || nb <= 0 || !dims) return MOSE_ERR_ARG;
   c.sc = *sc;
   c.nprim = sc->nsc + 4 + sc->nrans;
-  int64_t NC = 0, NF = 0, NFI[3] = {0, 0, 0}, NBP = 0;
+  c.blk.resize(nb);
+  int64_t NC = 0, NF = 0, NFI[3] = {0, 0, 0}, NBP = 0, tiles = 0;
   for (int b = 0; b < nb; ++b) {
     int64_t n1 = dims[3 * b], n2 = dims[3 * b + 1], n3 = dims[3 * b + 2];
     NC += (n1 + 4) * (n2 + 4) * (n3 + 4);
     NF += (n1 + 1) * n2 * n3 + n1 * (n2 + 1) * n3 + n1 * n2 * (n3 + 1);
     NFI[0] += (n1 - 1) * n2 * n3; NFI[1] += n1 * (n2 - 1) * n3; NFI[2] += n1 * n2 * (n3 - 1);
     NBP += 2 * (n2 * n3 + n1 * n3 + n1 * n2);
+    tiles += ((n1 + 7) / 8) * ((n2 + 3) / 4) * ((n3 + 3) / 4);
   }
   c.NC = NC; c.NF1 = NF; c.NF2 = 0; c.NF3 = 0; c.NBP = NBP;
   for (int d = 0; d < 3; ++d) c.NFI[d] = std::max<int64_t>(NFI[d], 1);
-  c.blk.resize(nb);
   c.rec.resize(std::max(nrec, 0));
-  *bytes = (int64_t)case_bytes(c);
+  *bytes = page_bytes(case_bytes(c) + kHistCap * sizeof(double)) + page_bytes(plan_bytes(c)) +
+           page_bytes((size_t)tiles * (c.nprim - c.sc.nsc + 1) * sizeof(double)) + page_bytes((size_t)tiles * sizeof(Tile));
   return MOSE_OK;
 }
 
 static int alloc_case(mose_ctx* ctx, Case& c) {
   size_t d = sizeof(double);
-  c.hist_cap = 4096;
+  c.hist_cap = kHistCap;
   size_t total = case_bytes(c) + (size_t)c.hist_cap * d;
   HIPCHK(ctx, hipMalloc(&c.slab, total));
   c.slab_bytes = total;
