@@ -16,10 +16,10 @@
 #include <memory>
 #include <mutex>
 #include <string>
-#include <thread>
 #include <vector>
 
 #include "mose_gpu.h"
+#include "mose_host.hpp"
 #include "mose_internal.h"
 #include "mose_chem.hpp"
 #include "mose_bc.hpp"
@@ -437,16 +437,6 @@ static bool bc_dead(const Case& c, const mose_bc_record& r) {
   const mose_blk& B = c.blk[r.b];
   const int d = (r.f + 1) / 2;
   return !c.sc.viscous && r.typ == MOSE_BC_NONE && (d == 1 ? B.n1 : (d == 2 ? B.n2 : B.n3)) == 1;
-}
-
-// f(first, last) over [0, n) in the host's threads (the plan of a large case: 0.3 us a record)
-template <class F>
-static void host_parallel(size_t n, F f) {
-  const size_t parts = n < 32768 ? 1 : std::min<size_t>(8, std::max(1u, std::thread::hardware_concurrency()));
-  std::vector<std::thread> th;
-  for (size_t t = 1; t < parts; ++t) th.emplace_back(f, n * t / parts, n * (t + 1) / parts);
-  f((size_t)0, n / parts);
-  for (auto& t : th) t.join();
 }
 
 static CaseDev make_dev(mose_ctx* ctx, Case& c, const double* Pin, double* Pout);
