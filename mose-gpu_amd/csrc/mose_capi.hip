@@ -423,7 +423,7 @@ static size_t case_bytes(const Case& c) {
 // the boundary plan, an allocation of its own that plan_boundary makes to size: at most this (without the records: dead
 // ones are not planned, some cases make no plan)
 static size_t plan_bytes(const Case& c) {
-  if (c.sc.nsc > 4) return 0;
+  if (c.sc.nsc > 4 || c.sc.irs) return 0;
   const size_t d = sizeof(double);
   if (!c.sc.viscous) return c.rec.size() * (sizeof(BcPlan) + BCG_INVISCID * d) + 256;
   return c.rec.size() * (sizeof(BcPlan) + sizeof(BcNbr) + BCG_VISCOUS * d) + (size_t)c.NBP * sizeof(int) + 256;
@@ -442,14 +442,15 @@ static bool bc_dead(const Case& c, const mose_bc_record& r) {
 static CaseDev make_dev(mose_ctx* ctx, Case& c, const double* Pin, double* Pout);
 static inline unsigned nblocks(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
 
-// The boundary plan (mose_bc.hpp).  Cases of nine species and connections whose transverse maps are not one step along
-// one axis keep k_ghost and k_bcrec (ghost1 forms the first ghost layer next to a cell, no corner).  So do cases with a
-// symmetry record or the receiver of a connection in a direction of one cell: their increments take the neighbour along
-// the normal, which there is the ghost behind the opposite face, and only the order of the two kernels gives them that
-// face's ghost of this stage.  (Walls and far-field faces need more cells along their normal, plan_case; extrapolation
-// and no-flux increments do not read the neighbour.)
+// The boundary plan (mose_bc.hpp).  Cases with residual smoothing run the plain path only and make none.  Cases of nine
+// species and connections whose transverse maps are not one step along one axis keep k_ghost and k_bcrec (ghost1 forms the
+// first ghost layer next to a cell, no corner).  So do cases with a symmetry record or the receiver
+// of a connection in a direction of one cell: their increments take the neighbour along the normal, which there is the
+// ghost behind the opposite face, and only the order of the two kernels gives them that face's ghost of this stage.
+// (Walls and far-field faces need more cells along their normal, plan_case; extrapolation and no-flux increments do not
+// read the neighbour.)
 static int plan_boundary(mose_ctx* ctx, Case& c, hipStream_t s) {
-  if (c.sc.nsc > 4 || c.rec.empty() || c.NC > 0x7fffffff || std::max({c.NF1, c.NF2, c.NF3, c.NBP}) > 0x7fffffff) return MOSE_OK;
+  if (c.sc.nsc > 4 || c.sc.irs || c.rec.empty() || c.NC > 0x7fffffff || std::max({c.NF1, c.NF2, c.NF3, c.NBP}) > 0x7fffffff) return MOSE_OK;
   auto row_of = [&](int b, const int* x) {
     const mose_blk& B = c.blk[b];
     return B.boff + (x[0] + MOSE_GC - 1) + (int64_t)(x[1] + MOSE_GC - 1) * B.pi + (int64_t)(x[2] + MOSE_GC - 1) * B.pi * B.pj;

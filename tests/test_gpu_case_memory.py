@@ -35,3 +35,15 @@ def test_unplanned_records_take_nothing(gpu_ready):
     got, stated = taken(case), serve.case_bytes(case)
     print(f"case memory: {got} B taken, {stated} B stated", flush=True)
     assert got <= stated - (80 << 20)
+
+
+def test_plain_only_cases_plan_nothing(gpu_ready):
+    """Residual smoothing runs the plain path: no plan in the stated figure, nor in what is taken."""
+    case = cases.taylor_green(128, 1)
+    planned = serve.case_bytes(case)
+    case.scheme.irs, case.scheme.irs_beta, case.scheme.irs_njacobi = 1, 0.5, 2
+    smoothing = (5 + 2 * 5) * case.layout.NC * 8      # the residual and the two sweeps
+    got, stated = taken(case), serve.case_bytes(case)
+    print(f"case memory: {got} B taken, {stated} B stated", flush=True)
+    assert stated <= planned + smoothing - (18 << 20) + GRAIN
+    assert got <= stated
