@@ -704,7 +704,8 @@ static Case* get_case(mose_ctx* ctx, int id) {
   ((sc).nsc == 9 ? F<9, 0>(__VA_ARGS__) : (sc).nsc == 4 ? F<4, 0>(__VA_ARGS__)                          \
                                         : (sc).nrans == 0 ? F<1, 0>(__VA_ARGS__) : F<1, 1>(__VA_ARGS__))
 
-// The device code of a path's stage kernels, asked for ahead of the first step (stage_kernel_parity in mose_stage.hpp)
+// The device code of the stage kernels of the path that a case is tuned to, asked for ahead of its first step
+// (stage_kernel_parity in mose_stage.hpp)
 template <int NS, int NR>
 static int load_stage(mose_ctx* ctx, int path) {
   hipFuncAttributes a;
@@ -811,7 +812,6 @@ extern "C" int mose_case_create(mose_ctx* ctx, const mose_scheme* sc, int nb, co
   }
   HIPCHK(ctx, hipStreamSynchronize(s));
   rc = plan_boundary(ctx, *c, s);
-  if (rc == MOSE_OK && c->path != MOSE_PATH_PLAIN) rc = MOSE_DISPATCH(c->sc, load_stage, ctx, c->path);
   choose_default_tile(ctx, *c);
   // the norm partials of either path: growing them in the first step is a free (5 ms)
   if (rc == MOSE_OK) rc = ensure_rpart(ctx, *c, std::max(plain_parts(*c), tile_count(*c, c->TI, c->TJ, c->TK)));

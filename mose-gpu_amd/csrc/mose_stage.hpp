@@ -490,7 +490,7 @@ void launch_stage_fast(const CaseDev& D, const StageArgs& A, int rs, bool visc, 
                        hipStream_t s);
 
 // A kernel of each of those translation units: the runtime loads a unit's code when it first meets one of its kernels
-// (3 ms), and the host asks for it when a case is made or tuned rather than in its first step.
+// (3 ms, once per process), and the host asks for the chosen path's when a case is tuned rather than in its first step.
 template <int NS, int NR>
 const void* stage_kernel_parity();
 template <int NS, int NR>
