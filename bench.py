@@ -110,7 +110,7 @@ def chemistry_leg(ncell: int, cpu_cells: int, threads: int, radau_cells: int = 0
     out, hr, idid, nstep = dc.download()
     dc.destroy()
     ctx.close()
-    res = {"cells": ncell, "value": ncell / (rep.ms * 1e-3), "unit": "cells/s", "kernel": "k_chem (RODAS, a team of ns+1 "
+    res = {"cells": ncell, "value": ncell / (rep.ms * 1e-3), "unit": "cells/s", "kernel": "k_chem2 (RODAS, a team of ns+1 "
            "lanes per cell, persistent queue)", "kernel_ms": rep.ms, "wall_s": wall, "steps_mean": float(nstep.mean()),
            "steps_max": int(nstep.max()), "rhs_evals": int(rep.rhs_total), "failed": int((idid < 0).sum()),
            "workload": "H2-O2-N2 9 species, 17 Arrhenius + 2 Troe, 1 atm, T U[900,2500] K, phi U[0.5,2], "
@@ -159,7 +159,7 @@ def radau5_leg(M, st, cpu_cells: int, threads: int):
     dc.destroy()
     ctx.close()
     stalled = int((idid == -2).sum())
-    res = {"cells": n, "value": n / (rep.ms * 1e-3), "unit": "cells/s", "kernel": "k_radau (RADAU5, a team of ns+1 "
+    res = {"cells": n, "value": n / (rep.ms * 1e-3), "unit": "cells/s", "kernel": "k_radau2 (RADAU5, a team of ns+1 "
            "lanes per cell, persistent queue)", "kernel_ms": rep.ms, "steps_mean": float(nstep.mean()),
            "steps_max": int(nstep.max()), "stopped_at_nmax": stalled, "failed_other": int((idid < 0).sum()) - stalled,
            "steps_mean_completed": float(nstep[idid >= 0].mean()) if (idid >= 0).any() else None}

@@ -92,7 +92,7 @@ inline int chem_teams(long long ncell, int cus, int per_wave) {
   return t < 1 ? 1 : (t > per_wave ? per_wave : (int)t);
 }
 
-// one persistent launch of k_radau (radau5) or k_chem over the cells of A (mose_chem.hip)
+// one persistent launch of RADAU5 or RODAS over the cells of A, in the form that the mechanism takes (mose_chem.hip)
 void launch_chem(const ChemDev& M, ChemArgs A, bool radau5, int cus, hipStream_t s);
 
 __device__ __forceinline__ double ctab(const ChemDev& M, const double* t, int T1, double Td) {
@@ -931,8 +931,9 @@ __device__ __forceinline__ void chem_cells(const ChemDev& M, const ChemArgs& A) 
   }
 }
 
-// The general form at four waves per SIMD; the two-round form at two, where its 256 registers hold the lane's part of the
-// step without spills (at three waves 478 registers spill and 24,576 cells take 1,151 ms in place of 602).
+// The general form at four waves per SIMD (190 registers spill); the two-round form at two, where its 256 registers hold the
+// lane's part of the step but for two spilled ones (at three waves 478 registers spilled and 24,576 cells took 1,151 ms; they
+// take 566).
 template <int NS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_chem(ChemDev M, ChemArgs A) {
   chem_cells<NS, false>(M, A);
