@@ -1103,6 +1103,19 @@ static void launch_stage(Case& c, const CaseDev& D, hipStream_t s, double rkc, b
   else launch_stage_tiles<NS, NR>(D, A, c.sc.riemann, c.sc.viscous != 0, grid, lds, s);
 }
 
+// the interior cells of `src` to `dst`, a workgroup per tile
+static __global__ void __launch_bounds__(256) k_copy_tiles(const Tile* tiles, int TI, int TJ, int TK, const mose_blk* blk,
+                                                           const double* src, double* dst, int64_t NC, int np) {
+  const Tile tl = tiles[blockIdx.x];
+  const mose_blk B = blk[tl.b];
+  for (int q = threadIdx.x; q < TI * TJ * TK; q += 256) {
+    const int i = tl.i0 + q % TI, j = tl.j0 + q / TI % TJ, k = tl.k0 + q / (TI * TJ);
+    if (i > B.n1 || j > B.n2 || k > B.n3) continue;
+    const int64_t c0 = row(B, i, j, k);
+    for (int v = 0; v < np; ++v) dst[v * NC + c0] = src[v * NC + c0];
+  }
+}
+
 static int case_chem_launch(mose_ctx* ctx, Case& c, hipStream_t s);
 
 template <int NS, int NR>
@@ -1149,8 +1162,12 @@ static int run_steps(mose_ctx* ctx, Case& c, int nsteps) {
     // the other half.  Each substage starts from the state it finds (Copy_State: P0 is the base of its stages).
     for (int istr = 1; istr <= nstr; ++istr) {
       for (int irk = 1; irk <= nrk; ++irk) {
+        // a stage reads its input at its cells' neighbours too, so it cannot write to it: the one stage of a one-stage
+        // scheme, which would read and write P0, writes PA and is copied back (in the plain path the update alone reads
+        // neighbours, for the SA source)
+        const bool back = nrk == 1 && (fused || (NR > 0 && !c.sc.irs));
         double* in = irk == 1 ? c.P0 : (irk == 2 ? c.PA : c.PB);
-        double* out = irk == nrk ? c.P0 : (irk == 1 ? c.PA : c.PB);
+        double* out = irk == nrk && !back ? c.P0 : (irk == 1 ? c.PA : c.PB);
         CaseDev D = make_dev(ctx, c, in, out);
         double rkc = rk[nrk - 1][irk - 1];
         const bool last = irk == nrk && istr == nstr;   // the step's last stage: next dt and the norm partials
@@ -1160,6 +1177,8 @@ static int run_steps(mose_ctx* ctx, Case& c, int nsteps) {
           launch_stage<NS, NR>(c, D, s, rkc, last);
           if (last) c.nparts_last = c.ntiles;
           if (c.timing) HIPCHK(ctx, hipEventRecord(c.tev[iev++], s));
+          if (back)
+            k_copy_tiles<<<(unsigned)c.ntiles, 256, 0, s>>>(c.dtiles, c.TI, c.TJ, c.TK, c.dblk, out, c.P0, c.NC, c.nprim);
         } else {
           launch_flux<NS, NR>(c, D, s);
           if (c.sc.irs) launch_irs<NS, NR>(c, D, s);
@@ -1173,6 +1192,10 @@ static int run_steps(mose_ctx* ctx, Case& c, int nsteps) {
           }
           if (last) c.nparts_last = part0;
           if (c.timing) HIPCHK(ctx, hipEventRecord(c.tev[iev++], s));
+          for (int b = 0; back && b < c.nb; ++b) {
+            const int64_t ncell = (int64_t)c.blk[b].n1 * c.blk[b].n2 * c.blk[b].n3;
+            k_irs_copy_interior<<<nblocks(ncell, 256), 256, 0, s>>>(c.blk[b], out, c.P0, c.NC, c.nprim);
+          }
         }
       }
       if (istr == 1 && nstr == 2) {
